@@ -406,4 +406,15 @@ template <class T, class OP> __device__ __forceinline__ T wave_allreduce(T v, OP
     return op(a, b);
 }
 
+// op over aligned groups of GL lanes (16 or 64), the result in every lane of the
+// group: wave_allreduce, or its first four steps, which stay inside 16 lanes.
+template <int GL, class T, class OP> __device__ __forceinline__ T lanes_allreduce(T v, OP op) {
+    static_assert(GL == 16 || GL == 64, "lane groups of 16 or 64");
+    if constexpr (GL == 64) return wave_allreduce(v, op);
+    v = op(v, dpp_mov<0xB1>(v));
+    v = op(v, dpp_mov<0x4E>(v));
+    v = op(v, dpp_mov<0x141>(v));
+    return op(v, dpp_mov<0x140>(v));
+}
+
 }  // namespace tohip

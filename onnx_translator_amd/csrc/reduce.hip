@@ -4,15 +4,20 @@
 // [outer, L, inner] around the axis; per (outer, inner) column the reference
 // takes the max over the axis (from -DBL_MAX), sums exp(v - max) in double and
 // writes exp(v - max) / sum.  Kernels here:
-//   * many rows (inner == 1): one 1024-thread block per row, the row held in
-//     registers, wave64 shuffle + LDS reductions, read once / written once;
+//   * rows of at most 512 values (inner == 1), many or short: a wave (16 lanes
+//     for rows of at most 32 values) per row, the row in registers, reductions
+//     by DPP moves and permlane swaps alone;
+//   * other rows (inner == 1): one block of 256 or 1024 threads per row, the row
+//     held in registers, wave64 shuffle + LDS reductions, read once / written once;
 //   * few long rows (inner == 1, e.g. [64, 32000]): each row is split over G
 //     blocks so the fp64 exp / divide work covers the chip: pass 1 writes each
 //     block's (max m_b, sum_b exp(v - m_b)); pass 2 folds them into the row's
 //     max M and sum S = sum_b s_b * exp(m_b - M) (fixed order) and writes
 //     exp(v - m_b) * (exp(m_b - M) / S); the one-launch form keeps exp(v - m_b)
 //     in registers from its partial pass, so each value is exponentiated once;
-//   * inner > 1: one thread per column, coalesced along the inner dimension.
+//   * inner > 1: a block takes 32 columns, its 32 rows of threads sharing each
+//     column's values (held in registers up to 512 of them), coalesced along
+//     the inner dimension.
 // Max, sums and the final scaling are in double (the sums are trees instead of the
 // reference's sequential loop); exp is sm_exp below (fp64 range reduction,
 // fp32 core) and the divide is a multiply by 1 / sum, so outputs agree with
@@ -28,6 +33,7 @@
 // window has a block-per-plane strip kernel that loads each input row once.
 #include <atomic>
 #include <cfloat>
+#include <type_traits>
 
 #include "quant.h"
 #include "runtime.h"
@@ -57,22 +63,22 @@ constexpr int kWaves = kRowThreads / 64;
 
 // Max (strict >) or sum over the wave's 64 lanes, the same result in every
 // lane (wave_allreduce: DPP moves and permlane swaps, all 64 lanes active).
-template <bool MAX> __device__ __forceinline__ double wave_reduce(double v) {
-    return wave_allreduce(v, [](double x, double y) { return MAX ? (y > x ? y : x) : x + y; });
+template <bool MAX, class T> __device__ __forceinline__ T wave_reduce(T v) {
+    return wave_allreduce(v, [](T x, T y) { return MAX ? (y > x ? y : x) : x + y; });
 }
 __device__ __forceinline__ double wave_max(double v) { return wave_reduce<true>(v); }
 __device__ __forceinline__ double wave_sum(double v) { return wave_reduce<false>(v); }
 
 // Block-wide reduction across the NW waves of a block (NW * 64 threads).
-template <bool MAX, int NW> __device__ __forceinline__ double block_reduce(double v, double* lds) {
-    v = MAX ? wave_max(v) : wave_sum(v);
+template <bool MAX, int NW, class T> __device__ __forceinline__ T block_reduce(T v, T* lds) {
+    v = wave_reduce<MAX>(v);
     const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
     if (l == 0) lds[w] = v;
     __syncthreads();
-    double r = lds[0];
+    T r = lds[0];
 #pragma unroll
     for (int i = 1; i < NW; i++) {
-        const double t = lds[i];
+        const T t = lds[i];
         r = MAX ? (t > r ? t : r) : r + t;
     }
     __syncthreads();
@@ -88,33 +94,57 @@ template <int DT> __device__ __forceinline__ void stx(void* p, int64_t i, double
     else st_d_rt(rdt, p, i, v);
 }
 
-// One block per row (inner == 1), the row kept in registers (IPT per thread).
-template <int IPT, int DIN, int DOUT>
-__global__ __launch_bounds__(kRowThreads) void k_softmax_row(const void* __restrict__ X, void* __restrict__ Y, int L) {
-    __shared__ double lds[kWaves];
-    const size_t base = (size_t)blockIdx.x * (size_t)L;
-    double v[IPT];
-    double mx = -DBL_MAX;
+// Output stores: nontemporal for f32, which is not read back here ([24576, 257]:
+// 12.4 -> 11.6 us).
+template <int DOUT> __device__ __forceinline__ void sm_store(void* Y, int64_t i, double v, int dty) {
+    if constexpr (DOUT == kF32) __builtin_nontemporal_store((float)v, (float*)Y + i);
+    else stx<DOUT>(Y, i, v, dty);
+}
+
+// A row's values in double: of a plain tensor, or (SmSlices, below) the k slices
+// of a Gemm.
+template <int DIN> struct SmRows {
+    // values that a float holds exactly are compared as floats
+    using T = std::conditional_t<DIN == kF32 || DIN == kF16, float, double>;
+    const void* X;
+    int dtx;
+    int64_t L;
+    __device__ __forceinline__ T operator()(int64_t row, int j) const { return (T)ldx<DIN>(X, row * L + j, dtx); }
+};
+
+// One block of T threads per row (inner == 1), the row kept in registers (IPT per
+// thread).
+template <int IPT, int T, int DOUT, class SRC>
+__global__ __launch_bounds__(T) void k_softmax_row(SRC src, void* __restrict__ Y, int dty, int L) {
+    constexpr int kW = T / 64;
+    using V = typename SRC::T;
+    const V kNone = (V)-__builtin_inf();
+    __shared__ V ldm[kW];
+    __shared__ double lds[kW];
+    const int64_t row = blockIdx.x;
+    V x[IPT], m = kNone;
 #pragma unroll
     for (int t = 0; t < IPT; t++) {
-        const int j = threadIdx.x + t * kRowThreads;
-        v[t] = j < L ? ld_d<DIN>(X, (int64_t)(base + j)) : -DBL_MAX;
-        mx = v[t] > mx ? v[t] : mx;
+        const int j = threadIdx.x + t * T;
+        x[t] = j < L ? src(row, j) : kNone;
+        m = x[t] > m ? x[t] : m;
     }
-    mx = block_reduce<true, kWaves>(mx, lds);
-    double sum = 0.0;
+    m = block_reduce<true, kW>(m, ldm);
+    // the reference's maximum starts at -DBL_MAX: what a row of -inf (or NaN) keeps
+    const double mx = m > kNone ? (double)m : -DBL_MAX;
+    double v[IPT], sum = 0.0;
 #pragma unroll
     for (int t = 0; t < IPT; t++) {
-        const int j = threadIdx.x + t * kRowThreads;
-        v[t] = j < L ? sm_exp(v[t] - mx) : 0.0;
+        const int j = threadIdx.x + t * T;
+        v[t] = j < L ? sm_exp((double)x[t] - mx) : 0.0;
         sum += v[t];
     }
-    sum = block_reduce<false, kWaves>(sum, lds);
+    sum = block_reduce<false, kW>(sum, lds);
     const double rs = 1.0 / sum;     // tolerance class: reciprocal instead of a divide per element
 #pragma unroll
     for (int t = 0; t < IPT; t++) {
-        const int j = threadIdx.x + t * kRowThreads;
-        if (j < L) st_d<DOUT>(Y, (int64_t)(base + j), v[t] * rs);
+        const int j = threadIdx.x + t * T;
+        if (j < L) sm_store<DOUT>(Y, row * L + j, v[t] * rs, dty);
     }
 }
 
@@ -457,37 +487,208 @@ bool launch_split(const void* x, int dtx, void* y, int dty, int64_t L, int G, di
     return launch_split_ipt<DIN, DOUT, 0>(x, dtx, y, dty, L, G, g, s);
 }
 
-// inner > 1: one thread per (outer, r) column; rows of the axis are coalesced across threads.
-__global__ __launch_bounds__(256) void k_softmax_cols(const void* __restrict__ X, int dtx, void* __restrict__ Y,
-                                                      int dty, int64_t L, int64_t inner) {
-    const int64_t r = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (r >= inner) return;
-    const int64_t base = (int64_t)blockIdx.y * L * inner + r;
+// inner > 1: CX columns (neighbours along the inner dimension: 128 or 256
+// contiguous bytes of f32 per row of threads) by CY rows of threads per block;
+// thread (c, r) holds values r, r + CY, ... of column c in registers (IPT of
+// them; 0: any number, read again in each of the three passes).  The CY partial
+// maxima and sums of a column meet in LDS and are folded in row order by every
+// thread.  One thread per column, the form before this, walked the axis three
+// times with dependent strided loads and left maps of few columns on a few CUs:
+// [8, 256, 1024] f32 241 -> 8.1 us, [4, 500, 16] 418 -> 8.6 us.  Axes of up to 64
+// values take 64 columns x 4 rows: 32 x 32 blocks would leave most rows of threads
+// one value or none ([64, 21, 4096]: 97 us, 12.3 us so).
+template <int IPT, int CX, int CY, int DIN, int DOUT>
+__global__ __launch_bounds__(CX * CY) void k_softmax_cols(const void* __restrict__ X, int dtx, void* __restrict__ Y,
+                                                               int dty, int64_t L, int64_t inner, uint32_t nbx) {
+    __shared__ double red[CY][CX];
+    const int cx = threadIdx.x & (CX - 1), ry = threadIdx.x / CX;
+    const int64_t bo = blockIdx.x / nbx;
+    const int64_t r = (int64_t)(blockIdx.x - bo * nbx) * CX + cx;
+    const bool live = r < inner;
+    const int64_t base = bo * L * inner + (live ? r : 0);
+    double v[IPT > 0 ? IPT : 1];
     double mx = -DBL_MAX;
-    for (int64_t j = 0; j < L; j++) {
-        const double v = ld_d_rt(dtx, X, base + j * inner);
-        mx = v > mx ? v : mx;
+    if constexpr (IPT > 0) {
+#pragma unroll
+        for (int t = 0; t < IPT; t++) {
+            const int64_t j = ry + (int64_t)t * CY;
+            v[t] = j < L ? ldx<DIN>(X, base + j * inner, dtx) : -DBL_MAX;
+        }
+#pragma unroll
+        for (int t = 0; t < IPT; t++) mx = v[t] > mx ? v[t] : mx;
+    } else {
+        for (int64_t j = ry; j < L; j += CY) {
+            const double w = ldx<DIN>(X, base + j * inner, dtx);
+            mx = w > mx ? w : mx;
+        }
     }
+    red[ry][cx] = mx;
+    __syncthreads();
+    mx = -DBL_MAX;
+#pragma unroll
+    for (int i = 0; i < CY; i++) {
+        const double w = red[i][cx];
+        mx = w > mx ? w : mx;
+    }
+    __syncthreads();
     double sum = 0.0;
-    for (int64_t j = 0; j < L; j++) sum += sm_exp(ld_d_rt(dtx, X, base + j * inner) - mx);
-    for (int64_t j = 0; j < L; j++) {
-        const int64_t i = base + j * inner;
-        st_d_rt(dty, Y, i, sm_exp(ld_d_rt(dtx, X, i) - mx) / sum);
+    if constexpr (IPT > 0) {
+#pragma unroll
+        for (int t = 0; t < IPT; t++) {
+            v[t] = ry + (int64_t)t * CY < L ? sm_exp(v[t] - mx) : 0.0;
+            sum += v[t];
+        }
+    } else {
+        for (int64_t j = ry; j < L; j += CY) sum += sm_exp(ldx<DIN>(X, base + j * inner, dtx) - mx);
+    }
+    red[ry][cx] = sum;
+    __syncthreads();
+    sum = 0.0;
+#pragma unroll
+    for (int i = 0; i < CY; i++) sum += red[i][cx];
+    if (!live) return;
+    const double rs = 1.0 / sum;
+    if constexpr (IPT > 0) {
+#pragma unroll
+        for (int t = 0; t < IPT; t++) {
+            const int64_t j = ry + (int64_t)t * CY;
+            if (j < L) stx<DOUT>(Y, base + j * inner, v[t] * rs, dty);
+        }
+    } else {
+        for (int64_t j = ry; j < L; j += CY)
+            stx<DOUT>(Y, base + j * inner, sm_exp(ldx<DIN>(X, base + j * inner, dtx) - mx) * rs, dty);
     }
 }
 
 template <int DIN, int DOUT>
-bool launch_row(const void* x, void* y, int64_t outer, int64_t L, hipStream_t s) {
-    const int ipt = (int)((L + kRowThreads - 1) / kRowThreads);
-    const dim3 g((unsigned)outer), b(kRowThreads);
-    const int Li = (int)L;
-    if (ipt <= 1) hipLaunchKernelGGL((k_softmax_row<1, DIN, DOUT>), g, b, 0, s, x, y, Li);
-    else if (ipt <= 2) hipLaunchKernelGGL((k_softmax_row<2, DIN, DOUT>), g, b, 0, s, x, y, Li);
-    else if (ipt <= 4) hipLaunchKernelGGL((k_softmax_row<4, DIN, DOUT>), g, b, 0, s, x, y, Li);
-    else if (ipt <= 8) hipLaunchKernelGGL((k_softmax_row<8, DIN, DOUT>), g, b, 0, s, x, y, Li);
-    else if (ipt <= 16) hipLaunchKernelGGL((k_softmax_row<16, DIN, DOUT>), g, b, 0, s, x, y, Li);
-    else if (ipt <= 32) hipLaunchKernelGGL((k_softmax_row<32, DIN, DOUT>), g, b, 0, s, x, y, Li);
+void launch_cols(const void* x, int dtx, void* y, int dty, int64_t outer, int64_t L, int64_t inner, hipStream_t s) {
+    const bool few = L <= 64;
+    const int cx = few ? 64 : 32, cy = few ? 4 : 32;
+    const uint32_t nbx = (uint32_t)((inner + cx - 1) / cx);
+    const int64_t ipt = (L + cy - 1) / cy;
+    const dim3 b(cx * cy);
+    // one grid dimension holds every (outer, column block): slices of at most 2^30 blocks
+    const int64_t per = std::max<int64_t>(1, ((int64_t)1 << 30) / nbx);
+    for (int64_t o = 0; o < outer; o += per) {
+        const dim3 g((unsigned)(std::min(per, outer - o) * nbx));
+        const char* xo = (const char*)x + (size_t)(o * L * inner) * dt_bytes(dtx);
+        char* yo = (char*)y + (size_t)(o * L * inner) * dt_bytes(dty);
+#define SM_COLS(I, CX, CY) \
+    hipLaunchKernelGGL((k_softmax_cols<I, CX, CY, DIN, DOUT>), g, b, 0, s, xo, dtx, yo, dty, L, inner, nbx)
+        if (few) {
+            if (ipt <= 2) SM_COLS(2, 64, 4);
+            else if (ipt <= 4) SM_COLS(4, 64, 4);
+            else if (ipt <= 8) SM_COLS(8, 64, 4);
+            else SM_COLS(16, 64, 4);
+        } else if (ipt <= 4) SM_COLS(4, 32, 32);
+        else if (ipt <= 8) SM_COLS(8, 32, 32);
+        else if (ipt <= 16) SM_COLS(16, 32, 32);
+        else SM_COLS(0, 32, 32);
+#undef SM_COLS
+    }
+}
+
+// Rows of at most 512 values (inner == 1): GL lanes per row (64, or 16 for rows
+// of at most 32 values), lane l holding values l, l + GL, ... (VPT of them) in
+// registers; the maximum and the sum are wave reductions, so a row needs no LDS
+// and no barrier, and a block's rows do not wait for each other.  What bounds it
+// is the memory traffic at 8 waves per SIMD.  One 1024-thread block per row, the
+// form before this, kept 1024 - L threads idle through two block-wide
+// reductions: [24576, 257] f32 107 -> 11.6 us (4.4 TB/s).
+template <int VPT, int GL, int DOUT, class SRC>
+__global__ __launch_bounds__(256) void k_softmax_wave(SRC src, void* __restrict__ Y, int dty, int64_t outer, int L) {
+    constexpr int kRows = 256 / GL;
+    using T = typename SRC::T;
+    const T kNone = (T)-__builtin_inf();
+    const int l = threadIdx.x & (GL - 1);
+    const int64_t row = (int64_t)blockIdx.x * kRows + threadIdx.x / GL;
+    const bool live = row < outer;              // (every lane takes part in the reductions)
+    T x[VPT], m = kNone;
+#pragma unroll
+    for (int t = 0; t < VPT; t++) {
+        const int j = l + t * GL;
+        x[t] = (live && j < L) ? src(row, j) : kNone;
+    }
+#pragma unroll
+    for (int t = 0; t < VPT; t++) m = x[t] > m ? x[t] : m;
+    m = lanes_allreduce<GL>(m, [](T a, T b) { return b > a ? b : a; });
+    // the reference's maximum starts at -DBL_MAX: what a row of -inf (or NaN) keeps
+    const double mx = m > kNone ? (double)m : -DBL_MAX;
+    double v[VPT], sum = 0.0;
+#pragma unroll
+    for (int t = 0; t < VPT; t++) {
+        v[t] = l + t * GL < L ? sm_exp((double)x[t] - mx) : 0.0;
+        sum += v[t];
+    }
+    sum = lanes_allreduce<GL>(sum, [](double a, double b) { return a + b; });
+    const double rs = 1.0 / sum;
+#pragma unroll
+    for (int t = 0; t < VPT; t++) {
+        const int j = l + t * GL;
+        if (live && j < L) sm_store<DOUT>(Y, row * L + j, v[t] * rs, dty);
+    }
+}
+
+// Which rows take k_softmax_wave: up to 256 values always (a block would idle most
+// of its threads); up to 512 when there are enough rows to fill the chip with one
+// wave each.  Fewer or longer ones spread better as a block each ([1024, 1000] 5.7
+// against 3.8 us, [8192, 1000] 15.4 against 12.0 us; [2048, 400] 3.8 against 3.8).
+inline bool sm_wave_rows(int64_t outer, int64_t L) {
+    return L <= 256 || (L <= 512 && outer >= 4 * (int64_t)num_cus());
+}
+
+template <int DOUT, class SRC>
+void launch_wave_rows(const SRC& src, void* y, int dty, int64_t outer, int L, hipStream_t s) {
+    const int vpt = (L + 63) / 64;
+    const dim3 b(256), g((unsigned)((outer + 3) / 4)), g16((unsigned)((outer + 15) / 16));
+#define SM_WAVE(V, G, GRID) hipLaunchKernelGGL((k_softmax_wave<V, G, DOUT, SRC>), GRID, b, 0, s, src, y, dty, outer, L)
+    if (L <= 16) SM_WAVE(1, 16, g16);
+    else if (L <= 32) SM_WAVE(2, 16, g16);
+    else if (vpt <= 1) SM_WAVE(1, 64, g);
+    else if (vpt <= 2) SM_WAVE(2, 64, g);
+    else if (vpt <= 3) SM_WAVE(3, 64, g);
+    else if (vpt <= 4) SM_WAVE(4, 64, g);
+    else if (vpt <= 5) SM_WAVE(5, 64, g);
+    else if (vpt <= 6) SM_WAVE(6, 64, g);
+    else SM_WAVE(8, 64, g);
+#undef SM_WAVE
+}
+
+// A block per row: T threads and values per thread by the row's length.
+template <int DOUT, class SRC>
+bool launch_block_rows(const SRC& src, void* y, int dty, int64_t outer, int L, hipStream_t s) {
+    const dim3 g((unsigned)outer);
+#define SM_ROW(I, T) hipLaunchKernelGGL((k_softmax_row<I, T, DOUT, SRC>), g, dim3(T), 0, s, src, y, dty, L)
+    // Many rows of at most 4096 values: 256 threads per row, so that up to eight
+    // rows share a CU and one row's loads cover another's reductions (1024
+    // threads: two rows per CU, both often at a barrier): [4096, 2000] 27.5 ->
+    // 11.0 us, [700, 700] 5.5 -> 3.7 us; at [600, 4096] the two forms took 9.2 and
+    // 9.5 us, so the longer rows only with four of them per CU.
+    if (L <= 4096 && outer >= (L <= 2048 ? 2 : 4) * num_cus()) {
+        if (L <= 1024) SM_ROW(4, 256);
+        else if (L <= 2048) SM_ROW(8, 256);
+        else SM_ROW(16, 256);
+        return true;
+    }
+    const int ipt = (L + kRowThreads - 1) / kRowThreads;
+    if (ipt <= 1) SM_ROW(1, kRowThreads);
+    else if (ipt <= 2) SM_ROW(2, kRowThreads);
+    else if (ipt <= 4) SM_ROW(4, kRowThreads);
+    else if (ipt <= 8) SM_ROW(8, kRowThreads);
+    else if (ipt <= 16) SM_ROW(16, kRowThreads);
+    else if (ipt <= 32) SM_ROW(32, kRowThreads);
     else return false;
+#undef SM_ROW
+    return true;
+}
+
+// Rows (inner == 1) that fit in registers; false: longer ones.  gemm_softmax_forward
+// takes the same way with the Gemm's slices as the source, so it sums in the same
+// order.
+template <int DOUT, class SRC>
+bool launch_rows(const SRC& src, void* y, int dty, int64_t outer, int L, hipStream_t s) {
+    if (!sm_wave_rows(outer, L)) return launch_block_rows<DOUT>(src, y, dty, outer, L, s);
+    launch_wave_rows<DOUT>(src, y, dty, outer, L, s);
     return true;
 }
 
@@ -733,47 +934,41 @@ __global__ __launch_bounds__(kGapSmallThreads) void k_gap_small_f32(const float*
     }
 }
 
-// Gemm -> Softmax (last axis) with the Gemm's k split: one block per row adds
-// the row's slice sums and the bias as k_splitk_reduce does (double sum in
-// slice order, alpha * acc + beta * c, rounded to f32), writes the logits, and
-// takes the row's softmax as k_softmax_row<1> does (max from -DBL_MAX with a
-// strict >, sm_exp, the block sums, one reciprocal): both outputs equal the
-// two launches they replace bit for bit.  cmode: 0 no bias, 1 one value, 2 per
-// column, 3 per row.  N <= kRowThreads.
-__global__ __launch_bounds__(kRowThreads) void k_splitk_softmax(const float* __restrict__ part, int nsplit, int M,
-                                                                int N, double alpha, double beta,
-                                                                const float* __restrict__ c, int cmode,
-                                                                float* __restrict__ Y, float* __restrict__ P) {
-    __shared__ double lds[kWaves];
-    const int m = blockIdx.x, j = threadIdx.x;
-    const int64_t mn = (int64_t)M * N, i = (int64_t)m * N + j;
-    double v = -DBL_MAX;
-    if (j < N) {
+// Gemm -> Softmax (last axis) with the Gemm's k split: the softmax kernels above
+// over the slices.  A value is the slices' sum and the bias as k_splitk_reduce
+// takes them (double sum in slice order, alpha * acc + beta * c, rounded to f32),
+// written to Y as the logit; the rows then run as softmax_forward runs them: both
+// outputs equal the two launches they replace bit for bit.  cmode: 0 no bias, 1
+// one value, 2 per column, 3 per row.
+struct SmSlices {
+    const float* part;
+    int nsplit;
+    int64_t mn;
+    int N;
+    double alpha, beta;
+    const float* c;
+    int cmode;
+    float* Y;
+    using T = float;
+    __device__ __forceinline__ float operator()(int64_t m, int j) const {
+        const int64_t i = m * N + j;
         double acc = 0.0;
         for (int sp = 0; sp < nsplit; sp++) acc += (double)part[(int64_t)sp * mn + i];
         double r = alpha * acc;
-        if (cmode) r += beta * (double)c[cmode == 1 ? 0 : (cmode == 2 ? j : m)];
+        if (cmode) r += beta * (double)c[cmode == 1 ? 0 : (cmode == 2 ? j : (int)m)];
         const float y = (float)r;
         Y[i] = y;
-        v = (double)y;
+        return y;
     }
-    double mx = -DBL_MAX;
-    mx = v > mx ? v : mx;
-    mx = block_reduce<true, kWaves>(mx, lds);
-    const double e = j < N ? sm_exp(v - mx) : 0.0;
-    const double sum = block_reduce<false, kWaves>(e, lds);
-    const double rs = 1.0 / sum;
-    if (j < N) P[i] = (float)(e * rs);
-}
+};
 
 }  // namespace
 
 bool launch_splitk_softmax(const float* part, int nsplit, int M, int N, double alpha, double beta, const float* c,
                            int cmode, float* Y, float* P, hipStream_t s) {
     if (N < 1 || N > kRowThreads || M < 1 || cmode < 0 || cmode > 3) return false;
-    hipLaunchKernelGGL(k_splitk_softmax, dim3((unsigned)M), dim3(kRowThreads), 0, s, part, nsplit, M, N, alpha, beta, c,
-                       cmode, Y, P);
-    return true;
+    const SmSlices src{part, nsplit, (int64_t)M * N, N, alpha, beta, c, cmode, Y};
+    return launch_rows<kF32>(src, P, kF32, M, N, s);
 }
 
 // Resolves sm_capture_ws on the library's device (current during initialisation).
@@ -863,15 +1058,21 @@ void softmax_forward(const Tensor* input, Tensor* output, int axis) {
         } else if (inner == 1) {
             bool done = false;
             if (outer <= 0x7FFFFFFF && L <= 0x7FFFFFFF) {
-                if (dtx == kF32 && dty == kF32) done = launch_row<kF32, kF32>(x, y, outer, L, s);
-                else if (dtx == kF16 && dty == kF16) done = launch_row<kF16, kF16>(x, y, outer, L, s);
-                else if (dtx == kF32 && dty == kF64) done = launch_row<kF32, kF64>(x, y, outer, L, s);
+                const int Li = (int)L;
+                if (dtx == kF32 && dty == kF32) done = launch_rows<kF32>(SmRows<kF32>{x, dtx, L}, y, dty, outer, Li, s);
+                else if (dtx == kF16 && dty == kF16) done = launch_rows<kF16>(SmRows<kF16>{x, dtx, L}, y, dty, outer, Li, s);
+                else if (dtx == kF32 && dty == kF64) done = launch_rows<kF64>(SmRows<kF32>{x, dtx, L}, y, dty, outer, Li, s);
+                else if (sm_wave_rows(outer, L)) {
+                    launch_wave_rows<-1>(SmRows<-1>{x, dtx, L}, y, dty, outer, Li, s);
+                    done = true;
+                }
             }
             if (!done)
                 hipLaunchKernelGGL(k_softmax_row_rt, dim3((unsigned)outer), dim3(kRowThreads), 0, s, x, dtx, y, dty, L);
         } else {
-            const dim3 g((unsigned)((inner + 255) / 256), (unsigned)outer);
-            hipLaunchKernelGGL(k_softmax_cols, g, dim3(256), 0, s, x, dtx, y, dty, L, inner);
+            if (dtx == kF32 && dty == kF32) launch_cols<kF32, kF32>(x, dtx, y, dty, outer, L, inner, s);
+            else if (dtx == kF16 && dty == kF16) launch_cols<kF16, kF16>(x, dtx, y, dty, outer, L, inner, s);
+            else launch_cols<-1, -1>(x, dtx, y, dty, outer, L, inner, s);
         }
         if (!check_launch(name)) { st.finish(); return; }
     }

@@ -10,6 +10,7 @@
 //    (c, kh, kw), MODE 1 1x1 float4, MODE 2 tap-blocked channels with
 //    b128 LDS reads), split-K for small grids, fused Relu / residual
 //    epilogue (described at the kernel and at launch_conv_tiled_xq).
+//  * convdw.hip — one input channel per group (depthwise), f32 or f16.
 //  * k_conv_mfma_f32 — other fp32-exact dtypes (decoded while staging):
 //    implicit GEMM on v_mfma_f32_32x32x2f32.  Per group:
 //    M = out channels, N = batch * OH * OW pixels, K = Cin/g * KH * KW.  The
@@ -22,21 +23,12 @@
 #include <algorithm>
 #include <cmath>
 
-#include "quant.h"
-#include "runtime.h"
+#include "conv.h"
 
 namespace tohip {
 namespace {
 
 typedef float floatx16 __attribute__((ext_vector_type(16)));
-
-struct ConvGeom {
-    int N, C, H, W;      // input
-    int M, KH, KW;       // weights [M, C/g, KH, KW]
-    int OH, OW;          // output (from Y)
-    int pt, pl, sh, sw, dh, dw, group;
-    int Cg, Mg, Kg;      // per-group channels in / out, Cg * KH * KW
-};
 
 __global__ __launch_bounds__(256) void k_conv_exact(const void* __restrict__ X, int dtx, const void* __restrict__ Wt,
                                                     int dtw, const void* __restrict__ Bv, int dtb, void* __restrict__ Y,
@@ -214,31 +206,6 @@ struct ConvTiled {
 };
 
 typedef __attribute__((address_space(1))) float gfloat;
-
-// Fused epilogue of conv2d_fused_forward (f32 output): y = conv + bias, then
-// Relu (v > 0 ? v : 0, as relu_forward), then + skip (an f32 tensor of Y's
-// shape, as add_forward).  Each step rounds to f32 exactly as the standalone
-// operator does, so the result equals the three calls bit for bit.
-struct ConvEpi {
-    const float* skip;
-    int relu;
-    FakeQuant fq;   // applied last (kind 0: none)
-};
-__device__ __forceinline__ float relu_f(float v) { return v > 0.0f ? v : 0.0f; }
-
-// Quantized input of dequantize_conv2d_fused_forward: X holds uint8 (XQ = 1) or
-// int8 (XQ = 2) codes with a per-tensor scale and zero point; the gather forms
-// (float)(q - z) * s, which is the value DequantizeLinear writes (q - z has at
-// most 9 bits, so the fp32 product is the correctly rounded exact product, as
-// the reference's double product rounded once).  Padding taps stay 0.
-struct ConvXQ {
-    const float* s;      // scale (one element)
-    const void* z;       // zero point of the codes' dtype (one element), or null for 0
-};
-template <int XQ> __device__ __forceinline__ float xq_value(uint32_t code, float s, int z) {
-    const int c = XQ == 2 ? (int)(int8_t)(uint8_t)code : (int)(code & 0xFFu);
-    return (float)(c - z) * s;
-}
 
 // SPLIT: gridDim.z = slices * groups, a block's z = slice * groups + group
 // (from its work index, below); slice s covers k in
@@ -1461,14 +1428,30 @@ bool conv_entry(const char* name, const Tensor* X, const Tensor* W, const Tensor
             const ConvEpi epi{(const float*)z, relu, fq};
             const ConvXQ xq{(const float*)xsd, xzd};
             bool fq_applied = false;
-            const bool ok = xq_kind == 1 ? launch_conv_tiled_xq<1>(x, w, b, dtb, y, dty, g, epi, xq, s, &fq_applied)
+            const bool dw = conv_depthwise_shape(g) &&
+                            launch_conv_depthwise(x, xq_kind == 1 ? kU8 : kI8, w, b, dtb, y, dty, g, epi, xq, s);
+            if (dw) fq_applied = fq_kind != 0;
+            const bool ok = dw ? true : xq_kind == 1 ? launch_conv_tiled_xq<1>(x, w, b, dtb, y, dty, g, epi, xq, s, &fq_applied)
                                          : launch_conv_tiled_xq<2>(x, w, b, dtb, y, dty, g, epi, xq, s, &fq_applied);
             if (!ok) set_error("%s: operands beyond the quantized-input kernel's reach", name);
             fused = true;
             if (fq_done) *fq_done = ok && fq_applied;
             done = true;
         } else if (!exact_mode() && !big && g.Kg > 0 && f32_exact_dtype(dtx) && f32_exact_dtype(dtw)) {
-            if (dtx == kF32 && dtw == kF32) {
+            const bool same = dtx == dtw && (dtx == kF32 || dtx == kF16);
+            const ConvEpi no_epi{nullptr, 0, FakeQuant{nullptr, nullptr, nullptr, nullptr, 0}};
+            if (same && conv_depthwise_shape(g)) {
+                const bool epi_ok = dty == kF32 && (!has_b || dtb == kF32);
+                const ConvEpi epi{(const float*)z, relu, fq};
+                if (launch_conv_depthwise(x, dtx, w, b, dtb, y, dty, g, epi_ok ? epi : no_epi,
+                                          ConvXQ{nullptr, nullptr}, s)) {
+                    fused = fused || epi_ok;
+                    if (fq_done) *fq_done = epi_ok && fq_kind != 0;
+                    done = true;
+                }
+            }
+            if (done) {
+            } else if (dtx == kF32 && dtw == kF32) {
                 const bool epi_ok = dty == kF32 && (!has_b || dtb == kF32);
                 const ConvEpi epi{epi_ok ? (const float*)z : nullptr, epi_ok ? relu : 0,
                                   epi_ok ? fq : FakeQuant{nullptr, nullptr, nullptr, nullptr, 0}};

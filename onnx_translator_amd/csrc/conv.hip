@@ -11,6 +11,7 @@
 //    b128 LDS reads), split-K for small grids, fused Relu / residual
 //    epilogue (described at the kernel and at launch_conv_tiled_xq).
 //  * convdw.hip — one input channel per group (depthwise), f32 or f16.
+//  * convh.hip — f16 input and weights on the f16 matrix cores.
 //  * k_conv_mfma_f32 — other fp32-exact dtypes (decoded while staging):
 //    implicit GEMM on v_mfma_f32_32x32x2f32.  Per group:
 //    M = out channels, N = batch * OH * OW pixels, K = Cin/g * KH * KW.  The
@@ -1450,6 +1451,7 @@ bool conv_entry(const char* name, const Tensor* X, const Tensor* W, const Tensor
                     done = true;
                 }
             }
+            if (!done && same && dtx == kF16) done = launch_conv_f16(x, w, b, dtb, y, dty, g, s);
             if (done) {
             } else if (dtx == kF32 && dtw == kF32) {
                 const bool epi_ok = dty == kF32 && (!has_b || dtb == kF32);

@@ -7,8 +7,7 @@
 // these layers before, gave a group's one channel a 64-channel tile.
 //
 // A block stages one tile of rows of a plane (or several small planes) in LDS as
-// f32, zero padding included, with every load of a thread issued before its first
-// LDS store; then a thread computes a strip of R output rows of one column, reading
+// f32, zero padding included (planes.h); then a thread computes a strip of R output rows of one column, reading
 // each input row of the strip once (K values) and adding it to the up to K outputs
 // that use it: (R - 1) S + K rows of K reads for R outputs instead of K K each.
 // The sum runs over (kh, kw) in the reference's order, in f32 with fused
@@ -18,31 +17,11 @@
 // stride 2 84 -> 11.7 us; the vector instructions and LDS reads of about 9 M
 // outputs, not only the traffic, bound the f16 form.  Output rows are stored plain:
 // nontemporal stores of rows that are no whole cache lines took 47 us.
-#include <algorithm>
-
 #include "conv.h"
+#include "planes.h"
 
 namespace tohip {
 namespace {
-
-constexpr int kDwThreads = 256;
-constexpr int kDwTile = 4096;        // floats of LDS tile aimed at: eight blocks or more per CU
-constexpr int kDwTileMax = 12288;    // and the most that a wide plane's shortest tile may take
-
-struct DwPlan {
-    int C, H, W, OH, OW, M;
-    int KH, KW, pt, pl, sh, sw, dh, dw;
-    int planes;          // N * M output planes
-    int np;              // planes per block (more than one only when a block holds whole planes)
-    int tiles;           // row tiles per plane
-    int TR;              // output rows per tile: ns strips
-    int ns;              // strips per tile
-    int PR, PW;          // LDS rows per plane and their pitch
-    int cc;              // column chunks of a row in the staging loop
-    int lxl, lxo;        // log2 of the threads along a row: staging, output
-    uint32_t xbytes;
-    FastDiv fd_tiles, fd_cc, fd_pr, fd_ns, fd_m, fd_mg;
-};
 
 // dec_f16's value (v_cvt_f32_f16 keeps f16 denormals; a NaN comes back quiet).
 __device__ __forceinline__ float f16_value(uint16_t h) { return (float)__builtin_bit_cast(_Float16, h); }
@@ -66,9 +45,9 @@ template <int DT> __device__ __forceinline__ float dw_wt(const void* w, int i) {
 // window, stride and dilation, R == 1.  MULTI: several planes per block.
 // FQ: the epilogue fake-quantizes (its fp64 fallback costs the other layers 10%).
 template <int DT, int ODT, int K, int S, int R, bool MULTI, bool FQ>
-__global__ __launch_bounds__(kDwThreads) void k_conv_dw(const void* __restrict__ X, const void* __restrict__ Wt,
+__global__ __launch_bounds__(kPlaneThreads) void k_conv_dw(const void* __restrict__ X, const void* __restrict__ Wt,
                                                         const void* __restrict__ Bv, int dtb, void* __restrict__ Y,
-                                                        DwPlan g, ConvEpi epi, ConvXQ xq) {
+                                                        PlaneTiles g, ConvEpi epi, ConvXQ xq) {
     extern __shared__ float tile[];
     constexpr int EB = DT == kF32 ? 4 : DT == kF16 ? 2 : 1;
     constexpr int KK = K > 0 ? K * K : 1;
@@ -85,85 +64,28 @@ __global__ __launch_bounds__(kDwThreads) void k_conv_dw(const void* __restrict__
         xs = xq.s[0];
         if (xq.z) xz = DT == kU8 ? (int)*(const uint8_t*)xq.z : (int)*(const int8_t*)xq.z;
     }
-    auto in_plane = [&](int p) {
-        if (g.M == g.C) return p;               // one output channel per input channel
-        const int n = (int)g.fd_m.div((uint32_t)p), m = p - n * g.M;
-        return n * g.C + (int)g.fd_mg.div((uint32_t)m);
-    };
-    auto channel = [&](int p) { return p - (int)g.fd_m.div((uint32_t)p) * g.M; };
-    // ---- stage the input rows (rows and columns outside the plane read zero)
-    {
-        const int lx = t & ((1 << g.lxl) - 1), ly = t >> g.lxl, step = kDwThreads >> g.lxl;
-        const int ih0 = tl * g.TR * (K > 0 ? S : g.sh) - g.pt;
-        constexpr int U = 8;
-        if constexpr (!MULTI) {
-            // one plane: a thread keeps its column; a row on is one addition to the
-            // load's and the LDS offset
-            const int rows0 = in_plane(p0) * g.H, ih_end = max(0, min(g.H, ih0 + g.PR));
-            for (int c = lx; c < g.PW; c += 1 << g.lxl) {
-                const int iw = c - g.pl;
-                const bool col = (unsigned)iw < (unsigned)g.W;
-                for (int r0 = ly; r0 < g.PR; r0 += step * U) {
-                    float v[U];
-                    uint32_t off = (uint32_t)((rows0 + ih0 + r0) * g.W + iw) * EB;
-#pragma unroll
-                    for (int u = 0; u < U; u++) {
-                        const int ih = ih0 + r0 + u * step;
-                        v[u] = dw_ld<DT>(xr, col && (unsigned)ih < (unsigned)ih_end ? off : kOOB, xs, xz);
-                        off += (uint32_t)(step * g.W) * EB;
-                    }
-                    float* to = tile + r0 * g.PW + c;
-#pragma unroll
-                    for (int u = 0; u < U; u++) {
-                        if (r0 + u * step < g.PR) *to = v[u];
-                        to += step * g.PW;
-                    }
-                }
-            }
-        } else {
-            const int items = np * g.PR * g.cc;
-            for (int i0 = ly; i0 < items; i0 += step * U) {
-                float v[U];
-                int at[U];
-#pragma unroll
-                for (int u = 0; u < U; u++) {
-                    const int i = i0 + u * step;
-                    const int rr = g.cc == 1 ? i : (int)g.fd_cc.div((uint32_t)i);
-                    const int c = ((i - rr * g.cc) << g.lxl) + lx;
-                    const int q = (int)g.fd_pr.div((uint32_t)rr);
-                    const int row0 = in_plane(min(p0 + q, g.planes - 1)) * g.H;
-                    const int ih = ih0 + rr - q * g.PR, iw = c - g.pl;
-                    const bool in = i < items && c < g.PW;
-                    const bool ok = in && (unsigned)ih < (unsigned)g.H && (unsigned)iw < (unsigned)g.W;
-                    at[u] = in ? rr * g.PW + c : -1;
-                    v[u] = dw_ld<DT>(xr, ok ? (uint32_t)((row0 + ih) * g.W + iw) * EB : kOOB, xs, xz);
-                }
-#pragma unroll
-                for (int u = 0; u < U; u++)
-                    if (at[u] >= 0) tile[at[u]] = v[u];
-            }
-        }
-    }
+    // rows and columns outside the plane read zero
+    stage_planes<EB, MULTI>(tile, g, tl, p0, np, [&](uint32_t off) { return dw_ld<DT>(xr, off, xs, xz); });
     if constexpr (MULTI) {
-        for (int i = t; i < np * kk; i += kDwThreads) {
+        for (int i = t; i < np * kk; i += kPlaneThreads) {
             const int q = i / kk;
-            wlds[i] = dw_wt<DT>(Wt, channel(p0 + q) * kk + (i - q * kk));
+            wlds[i] = dw_wt<DT>(Wt, g.channel(p0 + q) * kk + (i - q * kk));
         }
     }
     __syncthreads();
     // ---- strips of R output rows of one column
-    const int tx = t & ((1 << g.lxo) - 1), ty = t >> g.lxo, step = kDwThreads >> g.lxo;
+    const int tx = t & ((1 << g.lxo) - 1), ty = t >> g.lxo, step = kPlaneThreads >> g.lxo;
     FQParm fqp;
     if constexpr (FQ) fqp = fq_parm(epi.fq);
     float w[KK];
     if constexpr (!MULTI && K > 0) {
-        const int m = channel(p0);
+        const int m = g.channel(p0);
 #pragma unroll
         for (int i = 0; i < KK; i++) w[i] = dw_wt<DT>(Wt, m * KK + i);
     }
     for (int st = ty; st < np * g.ns; st += step) {
         const int q = MULTI ? (int)g.fd_ns.div((uint32_t)st) : 0;
-        const int strip = st - q * g.ns, p = p0 + q, m = channel(p);
+        const int strip = st - q * g.ns, p = p0 + q, m = g.channel(p);
         if constexpr (MULTI && K > 0) {
 #pragma unroll
             for (int i = 0; i < KK; i++) w[i] = wlds[q * KK + i];
@@ -218,22 +140,10 @@ __global__ __launch_bounds__(kDwThreads) void k_conv_dw(const void* __restrict__
     }
 }
 
-// Threads along a row of n elements (log2): the most, up to a wave, that leave at
-// most a quarter of them idle against the best of 16, 32 and 64 (8 for rows that
-// short): wide rows keep their loads and stores contiguous.
-int row_threads_log2(int n) {
-    if (n <= 8) return 3;
-    auto cost = [n](int l) { return (n + (1 << l) - 1) >> l << l; };
-    const int best = std::min(cost(4), std::min(cost(5), cost(6)));
-    for (int l = 6; l > 4; l--)
-        if (4 * cost(l) <= 5 * best) return l;
-    return 4;
-}
-
 template <int DT, int ODT, int K, int S, int R>
-void launch_dw(const void* x, const void* w, const void* b, int dtb, void* y, const DwPlan& p, const ConvEpi& epi,
+void launch_dw(const void* x, const void* w, const void* b, int dtb, void* y, const PlaneTiles& p, const ConvEpi& epi,
                const ConvXQ& xq, hipStream_t s) {
-    const dim3 grid((unsigned)((p.planes + p.np - 1) / p.np * p.tiles)), blk(kDwThreads);
+    const dim3 grid((unsigned)((p.planes + p.np - 1) / p.np * p.tiles)), blk(kPlaneThreads);
     const size_t lds = ((size_t)p.np * p.PR * p.PW + (p.np > 1 ? (size_t)p.np * p.KH * p.KW : 0)) * sizeof(float);
 #define DW_LAUNCH(MULTI, FQ) \
     hipLaunchKernelGGL((k_conv_dw<DT, ODT, K, S, R, MULTI, FQ>), grid, blk, lds, s, x, w, b, dtb, y, p, epi, xq)
@@ -256,7 +166,7 @@ constexpr int kDwR3 = 7, kDwR5 = 4;
 // channel, 3x3: 16 outputs 7.6 -> 4.6 us, 32 6.9 against 7.6, 64 10.9 against 11.4).
 constexpr int kDwMaxMult = 16;
 
-bool dw_plan(const ConvGeom& g, DwPlan& p) {
+bool dw_plan(const ConvGeom& g, PlaneTiles& p) {
     if (g.Cg != 1 || g.Mg > kDwMaxMult || g.KH < 1 || g.KW < 1 || g.sh < 1 || g.sw < 1 || g.dh < 1 || g.dw < 1) return false;
     const int64_t reach = (int64_t)1 << 29;              // elements: byte offsets stay below 2^31
     const int64_t planes = (int64_t)g.N * g.M;
@@ -265,41 +175,14 @@ bool dw_plan(const ConvGeom& g, DwPlan& p) {
     const bool strip = g.KH == g.KW && (g.KH == 3 || g.KH == 5) && g.sh == g.sw && (g.sh == 1 || g.sh == 2) &&
                        g.dh == 1 && g.dw == 1;
     const int R = strip ? (g.KH == 3 ? kDwR3 : kDwR5) : 1;
-    const int64_t pw = (int64_t)(g.OW - 1) * g.sw + (int64_t)(g.KW - 1) * g.dw + 1;
-    auto rows = [&](int64_t tr) { return (tr - 1) * g.sh + (int64_t)(g.KH - 1) * g.dh + 1; };
-    if (pw > kDwTileMax || rows(R) * pw > kDwTileMax) return false;
-    const int all = (g.OH + R - 1) / R;                  // strips of a plane
-    int ns = all;
-    while (ns > 1 && rows((int64_t)ns * R) * pw > kDwTile) ns--;
-    p.tiles = (all + ns - 1) / ns;
-    ns = (all + p.tiles - 1) / p.tiles;                  // even tiles
-    p.ns = ns;
-    p.TR = ns * R;
-    p.PR = (int)rows(p.TR);
-    p.PW = (int)pw;
-    p.np = 1;
-    if (p.tiles == 1) {
-        // several small planes per block, as long as two blocks per CU remain
-        const int64_t fit = kDwTile / ((int64_t)p.PR * p.PW + g.KH * g.KW);
-        p.np = (int)std::max<int64_t>(1, std::min<int64_t>(fit, planes / (2 * num_cus())));
-    }
     p.C = g.C; p.H = g.H; p.W = g.W; p.OH = g.OH; p.OW = g.OW; p.M = g.M; p.KH = g.KH; p.KW = g.KW;
     p.pt = g.pt; p.pl = g.pl; p.sh = g.sh; p.sw = g.sw; p.dh = g.dh; p.dw = g.dw;
     p.planes = (int)planes;
-    p.lxl = row_threads_log2(p.PW);
-    p.lxo = row_threads_log2(p.OW);
-    p.cc = (p.PW + (1 << p.lxl) - 1) >> p.lxl;
-    p.fd_tiles = make_fastdiv((uint32_t)p.tiles);
-    p.fd_cc = make_fastdiv((uint32_t)p.cc);
-    p.fd_pr = make_fastdiv((uint32_t)p.PR);
-    p.fd_ns = make_fastdiv((uint32_t)p.ns);
-    p.fd_m = make_fastdiv((uint32_t)g.M);
-    p.fd_mg = make_fastdiv((uint32_t)g.Mg);
-    return true;
+    return plan_planes(p, R, g.KH * g.KW);
 }
 
 template <int DT, int ODT>
-void launch_dw_window(const void* x, const void* w, const void* b, int dtb, void* y, const DwPlan& p, const ConvEpi& epi,
+void launch_dw_window(const void* x, const void* w, const void* b, int dtb, void* y, const PlaneTiles& p, const ConvEpi& epi,
                       const ConvXQ& xq, hipStream_t s) {
     const bool strip = p.KH == p.KW && p.sh == p.sw && p.sh <= 2 && p.dh == 1 && p.dw == 1;
     if (strip && p.KH == 3 && p.sh == 1) launch_dw<DT, ODT, 3, 1, kDwR3>(x, w, b, dtb, y, p, epi, xq, s);
@@ -312,7 +195,7 @@ void launch_dw_window(const void* x, const void* w, const void* b, int dtb, void
 }  // namespace
 
 bool conv_depthwise_shape(const ConvGeom& g) {
-    DwPlan p;
+    PlaneTiles p;
     return dw_plan(g, p);
 }
 
@@ -320,7 +203,7 @@ bool launch_conv_depthwise(const void* x, int dtx, const void* w, const void* b,
                            const ConvGeom& g, const ConvEpi& epi, const ConvXQ& xq, hipStream_t s) {
     const bool codes = dtx == kU8 || dtx == kI8;
     if ((dtx != kF32 && dtx != kF16 && !codes) || (codes && dty != kF32) || (dty != kF32 && dty != kF16) || (b && dtb != kF32 && dtb != kF16)) return false;
-    DwPlan p;
+    PlaneTiles p;
     if (!dw_plan(g, p)) return false;
     p.xbytes = (uint32_t)((int64_t)g.N * g.C * g.H * g.W * (codes ? 1 : dtx == kF16 ? 2 : 4));
     if (dtx == kU8) launch_dw_window<kU8, kF32>(x, w, b, dtb, y, p, epi, xq, s);

@@ -5,7 +5,7 @@
 // broadcast rules and writes through the output encoder.  Three kernels:
 //
 //  * k_gemm_mfma_f32 — v_mfma_f32_32x32x2f32 (fp32 operands, fp32 accumulate),
-//    for the layouts and dtypes k_gemm_f32_nt does not take.
+//    for the layouts (transA = 1) and dtypes k_gemm_f32_nt does not take.
 //    Operands of any dtype exactly representable in fp32 (f32, f16, bf16,
 //    fp8, int4/8/16, uint8) are decoded while staging into LDS.
 //    128x128 block tile, 4 waves (2x2), each wave 64x64 = 2x2 MFMA tiles,
@@ -15,8 +15,11 @@
 //    each), operands through raw buffer loads into registers one k-tile
 //    ahead, LDS double buffer, XCD-aware tile order.  fp32 accumulate.
 //  * k_gemm_f32_nt — f32 A [M, K] with B [N, K] of f32 or int8 / uint8 codes
-//    (dequantised while staging): v_mfma_f32_32x32x2f32, 128x256x16 tiles over
-//    8 waves, split-K with a deterministic reduction for small grids.
+//    (dequantised while staging) or f32 B [K, N]: v_mfma_f32_32x32x2f32,
+//    128x256x16 tiles over 8 waves, split-K with a deterministic reduction for
+//    small grids.
+//  * k_gemm_rows — the same operands with at most 64 rows of A and B [N, K]: one
+//    pass over B straight into the MFMA operands.
 //  * k_gemm_mfma_f16 — the other f16 transposes: 128x128x32 tiles.
 //  * k_gemm_exact — fp64, sequential k, no contraction: bit-identical to the
 //    reference for every dtype combination.  Used for f64 / int32 / int64
@@ -45,6 +48,13 @@ __device__ __forceinline__ u32x4 mask_k8(u32x4 v, int k, int K) {
         const uint32_t lo = (k + 2 * w < K) ? 0x0000FFFFu : 0u, hi = (k + 2 * w + 1 < K) ? 0xFFFF0000u : 0u;
         v[w] &= lo | hi;
     }
+    return v;
+}
+
+// Zero the elements of a 4-float chunk starting at k whose index is >= K.
+__device__ __forceinline__ u32x4 mask_k4(u32x4 v, int k, int K) {
+#pragma unroll
+    for (int w = 0; w < 4; w++) v[w] = k + w < K ? v[w] : 0u;
     return v;
 }
 
@@ -766,7 +776,18 @@ struct WoqB {
 // SPLIT: blockIdx.y takes k in [y * kchunk, (y + 1) * kchunk) (kchunk a
 // multiple of BK) and writes its raw fp32 sums to the workspace g.Y + y * M * N;
 // k_splitk_reduce adds the slices in order and applies the epilogue.
-template <int BM, int BN, int BK, int WGM, int WGN, int YDT, int BQ, int IGLP = -1, bool SPLIT = false>
+// KN: B is stored [K, N] (transB = 0), f32 only.  Its tile keeps that order in LDS, one
+// row of BN + 4 floats per k (lane halves then read rows 8 apart, 32 banks apart), and the
+// operand is one 4-byte read per MFMA and column tile instead of a 16-byte one per four:
+// little beside 64 cycles of f32 MFMA each, and the loads and LDS stores stay 16 bytes.
+// Rows need no alignment beyond a float's (buffer loads take 16 bytes at any 4-byte
+// address).  KT (K % 4 != 0): the elements of a last chunk past K are zeroed before they
+// are stored (in every instance that test took [512, 1024] x [4096, 1024] from 45.7 to
+// 52 us).  [512, 1024] x [1024, 4096] (KN) 124 -> 49.2 us, [300, 1003] x [1001, 1003] 329 ->
+// 22.1, [66, 3616] x [3616, 110] 674 -> 19.0 us against the 128x128 kernel without a k
+// split that took them before.
+template <int BM, int BN, int BK, int WGM, int WGN, int YDT, int BQ, int IGLP = -1, bool SPLIT = false, bool KN = false,
+          bool KT = false>
 __global__ __launch_bounds__(64 * WGM * WGN) void k_gemm_f32_nt(GemmArgs g, WoqB q, int kchunk) {
     constexpr int NT = 64 * WGM * WGN;
     constexpr int LDK = BK + 4;
@@ -777,7 +798,9 @@ __global__ __launch_bounds__(64 * WGM * WGN) void k_gemm_f32_nt(GemmArgs g, WoqB
     constexpr int EB = BQ ? 1 : 4;                // bytes per B element
     static_assert(CA * NT == BM * CPR && CB * NT == BN * CPR && CA >= 1 && CB >= 1, "tile / thread mismatch");
     static_assert(TM >= 1 && TN >= 1 && BK % 8 == 0, "wave tile");
-    __shared__ float lds[2][(BM + BN) * LDK];
+    constexpr int LDN = BN + 4, CPN = BN / 4;     // KN: row pitch and 4-element chunks per row of k
+    static_assert(!KN || !BQ, "codes are stored [N, K]");
+    __shared__ __attribute__((aligned(16))) float lds[2][KN ? BM * LDK + BK * LDN : (BM + BN) * LDK];
 
     const int nbm = (g.M + BM - 1) / BM, nbn = (g.N + BN - 1) / BN;
     int tm, tn;
@@ -787,7 +810,7 @@ __global__ __launch_bounds__(64 * WGM * WGN) void k_gemm_f32_nt(GemmArgs g, WoqB
     const int wm = wave / WGN, wn = wave % WGN;
     // Rows past M / N read as zero; the host guarantees (rows + tile) * ld * size < 2^31.
     const __amdgpu_buffer_rsrc_t ar = buffer_rsrc(g.A, (uint32_t)((int64_t)g.M * g.lda * 4));
-    const __amdgpu_buffer_rsrc_t br = buffer_rsrc(g.B, (uint32_t)((int64_t)g.N * g.ldb * EB));
+    const __amdgpu_buffer_rsrc_t br = buffer_rsrc(g.B, (uint32_t)((int64_t)(KN ? g.K : g.N) * g.ldb * EB));
 
     // Per-row dequantisation constants of the B chunks this thread stages
     // (a thread's chunk rows do not change across k-tiles).
@@ -816,6 +839,11 @@ __global__ __launch_bounds__(64 * WGM * WGN) void k_gemm_f32_nt(GemmArgs g, WoqB
 #pragma unroll
         for (int i = 0; i < CB; i++) {
             const int c = t + i * NT;
+            if constexpr (KN) {
+                const int k = k0 + c / CPN, n = n0 + (c % CPN) * 4;
+                rb[i] = ld_buf_b128(br, k < g.K && n < g.N ? (uint32_t)((k * g.ldb + n) * 4) : kOOB);
+                continue;
+            }
             const int k = k0 + (c % CPR) * 4;
             const uint32_t off = k < g.K ? (uint32_t)(((n0 + c / CPR) * g.ldb + k) * EB) : kOOB;
             if constexpr (BQ) rq[i] = __builtin_amdgcn_raw_buffer_load_b32(br, off, 0, 0);
@@ -823,6 +851,14 @@ __global__ __launch_bounds__(64 * WGM * WGN) void k_gemm_f32_nt(GemmArgs g, WoqB
         }
     };
     auto store_tile = [&](int buf, int k0) {
+        if (KT && k0 + BK > g.K) {
+#pragma unroll
+            for (int i = 0; i < CA; i++) ra[i] = mask_k4(ra[i], k0 + ((t + i * NT) % CPR) * 4, g.K);
+            if constexpr (!BQ && !KN) {
+#pragma unroll
+                for (int i = 0; i < CB; i++) rb[i] = mask_k4(rb[i], k0 + ((t + i * NT) % CPR) * 4, g.K);
+            }
+        }
 #pragma unroll
         for (int i = 0; i < CA; i++) {
             const int c = t + i * NT;
@@ -831,7 +867,8 @@ __global__ __launch_bounds__(64 * WGM * WGN) void k_gemm_f32_nt(GemmArgs g, WoqB
 #pragma unroll
         for (int i = 0; i < CB; i++) {
             const int c = t + i * NT;
-            float* dst = &lds[buf][(BM + c / CPR) * LDK + (c % CPR) * 4];
+            float* dst = KN ? &lds[buf][BM * LDK + (c / CPN) * LDN + (c % CPN) * 4]
+                            : &lds[buf][(BM + c / CPR) * LDK + (c % CPR) * 4];
             if constexpr (BQ) {
                 // Past K the A operand is zero, but (0 - zp) * s need not be: zero it.
                 const bool ok = k0 + (c % CPR) * 4 < g.K;
@@ -861,14 +898,21 @@ __global__ __launch_bounds__(64 * WGM * WGN) void k_gemm_f32_nt(GemmArgs g, WoqB
     const int lr = lane & 31, lh = (lane >> 5) * (BK / 2);
     auto compute = [&](int buf) {
         const float* As = &lds[buf][(wm * WTM + lr) * LDK + lh];
-        const float* Bs = &lds[buf][(BM + wn * WTN + lr) * LDK + lh];
+        const float* Bs = KN ? &lds[buf][BM * LDK + lh * LDN + wn * WTN + lr] : &lds[buf][(BM + wn * WTN + lr) * LDK + lh];
 #pragma unroll
         for (int s4 = 0; s4 < BK / 2; s4 += 4) {
             float4 a[TM], b[TN];
 #pragma unroll
             for (int i = 0; i < TM; i++) a[i] = *reinterpret_cast<const float4*>(As + i * 32 * LDK + s4);
 #pragma unroll
-            for (int j = 0; j < TN; j++) b[j] = *reinterpret_cast<const float4*>(Bs + j * 32 * LDK + s4);
+            for (int j = 0; j < TN; j++) {
+                if constexpr (KN) {
+                    const float* p = Bs + s4 * LDN + j * 32;
+                    b[j] = make_float4(p[0], p[LDN], p[2 * LDN], p[3 * LDN]);
+                } else {
+                    b[j] = *reinterpret_cast<const float4*>(Bs + j * 32 * LDK + s4);
+                }
+            }
 #pragma unroll
             for (int e = 0; e < 4; e++)
 #pragma unroll
@@ -928,6 +972,134 @@ __global__ __launch_bounds__(256) void k_splitk_reduce(GemmArgs g, const float* 
     for (int sp = 0; sp < nsplit; sp++) acc += (double)part[(int64_t)sp * mn + i];
     const int m = (int)fd_n.div((uint32_t)i);
     epilogue_fast<YDT>(g, m, i - m * g.N, acc);
+}
+
+// ------------------------------------------------------- few rows (NT, f32) ---
+// M <= 16 MT rows of f32 A against B [N, K] of f32 or int8 / uint8 codes: a batch too
+// small to fill a tile.  What bounds it is one pass over B (or, for codes, the MFMAs of
+// 16 padded rows: 3.4 us at N = K = 4096).  A block takes 16 columns of the output; its
+// waves take the 64-deep chunks of k in turn, each lane loading its row's 16 consecutive
+// k straight into registers (lane group h of four: k = 16 h ..; MFMA step e multiplies
+// k = 16 h + e in every group, A and B alike), so B is read once, without LDS, 64 (codes)
+// or 256 (f32) contiguous bytes of a row per wave and chunk (a second chunk in flight per
+// wave measured the same or slower: the other waves' loads are in flight anyway).  The
+// waves' sums meet in LDS and are added in wave order in double.  One launch, no workspace.  The order of the sums depends on K and the number
+// of waves (from N and K) only, and the codes' values are DequantizeLinear's bits (as in
+// k_gemm_f32_nt), so the fused and the unfused weight-only-quantized Gemm agree bit for
+// bit.  128-row tiles with a k split took these before: A [8, 4096] x int8 [4096, 4096]
+// 45 -> MEASW us.
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+
+template <int MT, int YDT, int BQ>
+__global__ __launch_bounds__(MT > 2 ? 512 : 1024) void k_gemm_rows(GemmArgs g, WoqB q) {
+    extern __shared__ float red[];            // [waves][16 MT][16]
+    const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int W = (int)blockDim.x >> 6, r = lane & 15, h = lane >> 4;
+    const int n0 = (int)blockIdx.x * 16, n = n0 + r;
+    constexpr int EB = BQ ? 1 : 4;
+    const __amdgpu_buffer_rsrc_t ar = buffer_rsrc(g.A, (uint32_t)((int64_t)g.M * g.lda * 4));
+    const __amdgpu_buffer_rsrc_t br = buffer_rsrc(g.B, (uint32_t)((int64_t)g.N * g.ldb * EB));
+    uint32_t arow[MT];
+#pragma unroll
+    for (int i = 0; i < MT; i++) arow[i] = r + 16 * i < g.M ? (uint32_t)(r + 16 * i) * (uint32_t)g.lda * 4u : kOOB;
+    const uint32_t brow = n < g.N ? (uint32_t)n * (uint32_t)g.ldb * EB : kOOB;
+    float bs = 0.0f, bz = 0.0f;               // int8 codes are read as code + 128
+    if constexpr (BQ) {
+        const int nc = min(n, g.N - 1), zi = q.zn > 1 ? nc : 0;
+        bs = q.s[q.per_n ? nc : 0];
+        const int z = q.zn == 0 ? 0 : (BQ == 1 ? (int)((const int8_t*)q.z)[zi] : (int)((const uint8_t*)q.z)[zi]);
+        bz = (float)(z + (BQ == 1 ? 128 : 0));
+    }
+    struct Chunk {
+        u32x4 a[MT][4];
+        u32x4 b[BQ ? 1 : 4];
+    };
+    // chunk c; in the last one a group of four k past K (K % 4 == 0) reads zeros
+    auto load = [&](Chunk& v, int c) {
+        const int k = c * 64 + 16 * h;
+        if (c * 64 + 64 <= g.K) {
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+#pragma unroll
+                for (int i = 0; i < MT; i++) v.a[i][j] = ld_buf_b128(ar, arow[i] + (uint32_t)k * 4u + 16u * j);
+                if constexpr (!BQ) v.b[j] = ld_buf_b128(br, brow + (uint32_t)k * 4u + 16u * j);
+            }
+            if constexpr (BQ) v.b[0] = ld_buf_b128(br, brow + (uint32_t)k);
+            return;
+        }
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const bool in = k + 4 * j < g.K;
+#pragma unroll
+            for (int i = 0; i < MT; i++) v.a[i][j] = ld_buf_b128(ar, in ? arow[i] + (uint32_t)(k + 4 * j) * 4u : kOOB);
+            if constexpr (BQ) v.b[0][j] = __builtin_amdgcn_raw_buffer_load_b32(br, in ? brow + (uint32_t)(k + 4 * j) : kOOB, 0, 0);
+            else v.b[j] = ld_buf_b128(br, in ? brow + (uint32_t)(k + 4 * j) * 4u : kOOB);
+        }
+    };
+    floatx4 acc[MT];
+#pragma unroll
+    for (int i = 0; i < MT; i++) acc[i] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+    auto multiply = [&](const Chunk& v, int c) {
+        // past K A is zero, but (0 - zp) * s need not be finite: the scale of a group past K is zero
+        const int k = c * 64 + 16 * h;
+        float sj[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) sj[j] = bs;
+        if (BQ && c * 64 + 64 > g.K) {
+#pragma unroll
+            for (int j = 0; j < 4; j++) sj[j] = k + 4 * j < g.K ? bs : 0.0f;
+        }
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const uint32_t w = BQ ? v.b[0][j] ^ (BQ == 1 ? 0x80808080u : 0u) : 0u;
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                float b;
+                if constexpr (BQ) {
+                    b = ((float)((w >> (8 * e)) & 255u) - bz) * sj[j];     // (an exact small integer) * s
+                } else {
+                    b = u2f(v.b[j][e]);
+                }
+#pragma unroll
+                for (int i = 0; i < MT; i++)
+                    acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(u2f(v.a[i][j][e]), b, acc[i], 0, 0, 0);
+            }
+        }
+    };
+    // the bias of this thread's (first) output, its latency under the loop's
+    const int o0 = t, m_o = o0 >> 4, n_o = n0 + (o0 & 15);
+    float c_o = 0.0f;
+    if constexpr (YDT == kF16 || YDT == kF32) {
+        if (g.c.mode && o0 < MT * 256 && m_o < g.M && n_o < g.N)
+            c_o = ((const gfloat*)g.c.p)[g.c.mode == 1 ? 0 : (g.c.mode == 2 ? n_o : m_o)];
+    }
+    const int nc = (g.K + 63) / 64;
+    for (int c = wave; c < nc; c += W) {
+        Chunk v;
+        load(v, c);
+        multiply(v, c);
+    }
+#pragma unroll
+    for (int i = 0; i < MT; i++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) red[((wave * MT + i) * 16 + 4 * h + e) * 16 + r] = acc[i][e];
+    __syncthreads();
+    for (int o = t; o < MT * 256; o += (int)blockDim.x) {
+        const int m = o >> 4, nn = n0 + (o & 15);
+        if (m >= g.M || nn >= g.N) continue;
+        double sum = 0.0;
+        for (int w = 0; w < W; w++) sum += (double)red[w * MT * 256 + o];
+        if constexpr (YDT == kF16 || YDT == kF32) {
+            if (o == o0) {                    // epilogue_fast with the bias at hand
+                double y = g.alpha * sum;
+                if (g.c.mode) y += g.beta * (double)c_o;
+                if constexpr (YDT == kF16) ((gu16*)g.Y)[(int64_t)m * g.N + nn] = enc_f16((float)y);
+                else ((gfloat*)g.Y)[(int64_t)m * g.N + nn] = (float)y;
+                continue;
+            }
+        }
+        epilogue_fast<YDT>(g, m, nn, sum);
+    }
 }
 
 // -------------------------------------------------------------------- dispatch ---
@@ -1011,36 +1183,74 @@ int nt_split_plan(int M, int N, int K, bool& big) {
     return (int)std::max<int64_t>(1, std::min<int64_t>(sp, 16));
 }
 
-template <int BM, int BN, int BK, int WGM, int WGN, int BQ, bool SPLIT>
-void launch_nt_kernel(const GemmArgs& g, const WoqB& q, int kchunk, int nsplit, int ydt, hipStream_t s) {
+template <int BM, int BN, int BK, int WGM, int WGN, int BQ, bool SPLIT, bool KN, bool KT>
+void launch_nt_kernel_kt(const GemmArgs& g, const WoqB& q, int kchunk, int nsplit, int ydt, hipStream_t s) {
     const dim3 grid(((g.M + BM - 1) / BM) * ((g.N + BN - 1) / BN), nsplit), block(64 * WGM * WGN);
     if (SPLIT || ydt == kF32)
-        hipLaunchKernelGGL((k_gemm_f32_nt<BM, BN, BK, WGM, WGN, kF32, BQ, -1, SPLIT>), grid, block, 0, s, g, q, kchunk);
+        hipLaunchKernelGGL((k_gemm_f32_nt<BM, BN, BK, WGM, WGN, kF32, BQ, -1, SPLIT, KN, KT>), grid, block, 0, s, g, q, kchunk);
     else if (ydt == kF16)
-        hipLaunchKernelGGL((k_gemm_f32_nt<BM, BN, BK, WGM, WGN, kF16, BQ, -1, SPLIT>), grid, block, 0, s, g, q, kchunk);
+        hipLaunchKernelGGL((k_gemm_f32_nt<BM, BN, BK, WGM, WGN, kF16, BQ, -1, SPLIT, KN, KT>), grid, block, 0, s, g, q, kchunk);
     else
-        hipLaunchKernelGGL((k_gemm_f32_nt<BM, BN, BK, WGM, WGN, -1, BQ, -1, SPLIT>), grid, block, 0, s, g, q, kchunk);
+        hipLaunchKernelGGL((k_gemm_f32_nt<BM, BN, BK, WGM, WGN, -1, BQ, -1, SPLIT, KN, KT>), grid, block, 0, s, g, q, kchunk);
+}
+
+template <int BM, int BN, int BK, int WGM, int WGN, int BQ, bool SPLIT, bool KN>
+void launch_nt_kernel(const GemmArgs& g, const WoqB& q, int kchunk, int nsplit, int ydt, hipStream_t s) {
+    if constexpr (BQ == 0) {
+        if (g.K & 3) {
+            launch_nt_kernel_kt<BM, BN, BK, WGM, WGN, BQ, SPLIT, KN, true>(g, q, kchunk, nsplit, ydt, s);
+            return;
+        }
+    }
+    launch_nt_kernel_kt<BM, BN, BK, WGM, WGN, BQ, SPLIT, KN, false>(g, q, kchunk, nsplit, ydt, s);
+}
+
+// Few rows: k_gemm_rows up to 32.  Up to 64 (four row tiles, 64 MFMAs per chunk and wave)
+// where the waves have few chunks each or the columns fill the chip; else the 128-row tiles
+// with their k split are as good: [64, 512] x [1000, 512] 10.5 -> 8.0 us, [48, 4096] x int8
+// [4096, 4096] 46.7 -> 29.5, but [64, 4096] x [4096, 4096] 42.3 against 43.1, [62, 4016] x
+// [344, 4016] 22.3 against 31.1.
+inline bool few_rows(int M, int N, int K) {
+    return M <= 32 || (M <= 64 && K <= 1024) || (M <= 48 && (N + 15) / 16 >= num_cus());
+}
+
+template <int MT, int BQ>
+void launch_rows_kernel(const GemmArgs& g, const WoqB& q, int ydt, hipStream_t s) {
+    const int nb = (g.N + 15) / 16, nc = (g.K + 63) / 64, wmax = MT > 2 ? 8 : 16;
+    const int W = std::max(1, std::min(nc, nb >= 2 * num_cus() ? std::min(8, wmax) : wmax));
+    const dim3 grid((unsigned)nb), block((unsigned)(64 * W));
+    const size_t lds = (size_t)W * MT * 256 * sizeof(float);
+    if (ydt == kF32) hipLaunchKernelGGL((k_gemm_rows<MT, kF32, BQ>), grid, block, lds, s, g, q);
+    else if (ydt == kF16) hipLaunchKernelGGL((k_gemm_rows<MT, kF16, BQ>), grid, block, lds, s, g, q);
+    else hipLaunchKernelGGL((k_gemm_rows<MT, -1, BQ>), grid, block, lds, s, g, q);
 }
 
 // probs (f32 [M, N], or null): with a k split, the reduction also takes the
 // rows' softmax into probs (returns 2); otherwise the caller runs the softmax.
-template <int BQ>
+// KN: B [K, N] (transB = 0).
+template <int BQ, bool KN = false>
 int launch_f32_nt(const GemmArgs& g, const WoqB& q, hipStream_t s, float* probs = nullptr) {
     const int64_t reach = (int64_t)1 << 31;
     const int eb = BQ ? 1 : 4;
-    if ((int64_t)(g.M + 256) * g.lda * 4 >= reach || (int64_t)(g.N + 256) * g.ldb * eb >= reach) return 0;
+    if ((int64_t)(g.M + 256) * g.lda * 4 >= reach || (int64_t)((KN ? g.K : g.N) + 256) * g.ldb * eb >= reach) return 0;
     const bool fast_bias = g.c.mode == 0 || (g.c.dt == kF32 && g.c.mode <= 3);
     const int ydt = fast_bias && (g.dty == kF32 || g.dty == kF16) ? g.dty : -1;
+    if (!KN && g.K % 4 == 0 && few_rows(g.M, g.N, g.K)) {
+        if (g.M <= 16) launch_rows_kernel<1, BQ>(g, q, ydt, s);
+        else if (g.M <= 32) launch_rows_kernel<2, BQ>(g, q, ydt, s);
+        else launch_rows_kernel<4, BQ>(g, q, ydt, s);
+        return 1;
+    }
     bool big = false;
     int split = nt_split_plan(g.M, g.N, g.K, big);
     // (no k split under graph capture: the slices' workspace would have to outlive the call)
     if (split > 1 && stream_capturing(s)) split = 1;
     if (big) {
-        launch_nt_kernel<128, 256, 16, 2, 4, BQ, false>(g, q, 0, 1, ydt, s);
+        launch_nt_kernel<128, 256, 16, 2, 4, BQ, false, KN>(g, q, 0, 1, ydt, s);
         return 1;
     }
     if (split <= 1) {
-        launch_nt_kernel<128, 64, 16, 2, 2, BQ, false>(g, q, 0, 1, ydt, s);
+        launch_nt_kernel<128, 64, 16, 2, 2, BQ, false, KN>(g, q, 0, 1, ydt, s);
         return 1;
     }
     const int kchunk = ((g.K + split - 1) / split + 15) / 16 * 16;
@@ -1050,7 +1260,7 @@ int launch_f32_nt(const GemmArgs& g, const WoqB& q, hipStream_t s, float* probs 
     if (!part) return -1;
     GemmArgs gp = g;
     gp.Y = part;
-    launch_nt_kernel<128, 64, 16, 2, 2, BQ, true>(gp, q, kchunk, nsplit, kF32, s);
+    launch_nt_kernel<128, 64, 16, 2, 2, BQ, true, KN>(gp, q, kchunk, nsplit, kF32, s);
     if (probs && ydt == kF32 &&
         launch_splitk_softmax(part, nsplit, g.M, g.N, g.alpha, g.beta, (const float*)g.c.p, g.c.mode, (float*)g.Y,
                               probs, s)) {
@@ -1148,9 +1358,10 @@ void gemm_impl(const char* name, const Tensor* A, const Tensor* B, const Tensor*
                 else launch_f16_y<true, false>(g, grid, vec, s);
                 done = true;
             } else if (f32_exact_dtype(dta) && f32_exact_dtype(dtb)) {
-                const bool nt = dta == kF32 && dtb == kF32 && !transA && transB && (g.lda % 4) == 0 &&
-                                (g.ldb % 4) == 0 && ((uintptr_t)g.A & 15) == 0 && ((uintptr_t)g.B & 15) == 0;
-                const int r = nt ? launch_f32_nt<0>(g, WoqB{nullptr, nullptr, 0, 0}, s, probs) : 0;
+                const bool tiled = dta == kF32 && dtb == kF32 && !transA && ((uintptr_t)g.A & 3) == 0 &&
+                                   ((uintptr_t)g.B & 3) == 0;
+                const WoqB f32_b{nullptr, nullptr, 0, 0};
+                const int r = !tiled ? 0 : transB ? launch_f32_nt<0>(g, f32_b, s, probs) : launch_f32_nt<0, true>(g, f32_b, s, probs);
                 if (r < 0) { st.finish(); return; }
                 if (r == 2 && softmax_done) *softmax_done = true;
                 done = r >= 1 || launch_f32_mfma(g, dta, dtb, transA, transB, s);

@@ -1273,9 +1273,18 @@ bool launch_conv_tiled_xq(const void* x, const void* w, const void* b, int dtb, 
         plan = kT64x256;
         no_split = true;
     }
-    const int bm = (plan == kT128x128 || plan == kT128x256) ? 128 : 64;
-    const int bp = (plan == kT64x128 || plan == kT128x128) ? 128 : 256;
-    const int64_t blocks = ((P + bp - 1) / bp) * ((g.Mg + bm - 1) / bm) * cg.group;
+    auto tiles = [&](int64_t bm, int64_t bp) { return ((P + bp - 1) / bp) * ((g.Mg + bm - 1) / bm) * cg.group; };
+    auto blocks_of = [&](int p) {
+        return tiles(p == kT128x128 || p == kT128x256 ? 128 : 64, p == kT64x128 || p == kT128x128 ? 128 : 256);
+    };
+    // A few images: grids that leave CUs idle even with the k range split (slices 128
+    // deep, at most 8) take the smallest tiles and up to 16 slices of 64: one image of
+    // the residual network's blocks 2-4 29.4 / 30.0 / 30.4 -> 12.2 / 14.0 / 16.6 us, two of
+    // [512, 7, 7] 3x3 53 -> 23.5.
+    const int64_t coarse = std::min<int64_t>(g.Kg / 128, 8);
+    const bool tiny = !direct && plan != kNone && blocks_of(plan) * std::max<int64_t>(1, coarse) < num_cus();
+    if (tiny) plan = kT64x128;
+    const int64_t blocks = blocks_of(plan);
     // Split-k slice count for grids smaller than the CU count: each slice
     // >= 128 deep, at most 8; the count whose block total balances best over
     // the CUs (fewer slices on near ties: each slice adds a write and a read of
@@ -1284,7 +1293,7 @@ bool launch_conv_tiled_xq(const void* x, const void* w, const void* b, int dtb, 
     int split = 1;
     // (not under graph capture: the slices' workspace would have to outlive the call)
     if (blocks < num_cus() && !no_split && !stream_capturing(s)) {
-        const int smax = (int)std::min<int64_t>(g.Kg / 128, 8);
+        const int smax = (int)(tiny ? std::min<int64_t>(g.Kg / 64, 16) : coarse);
         const double base = balance(blocks);
         double best = base;
         for (int sp = 2; sp <= smax; sp++) {

@@ -1103,8 +1103,25 @@ bool launch_splitk_softmax(const float* part, int nsplit, int M, int N, double a
     return launch_rows<kF32>(src, P, kF32, M, N, s);
 }
 
+namespace {
+template <class T>
+__global__ __launch_bounds__(256) void k_result(const T* __restrict__ src, T* __restrict__ dst, uint32_t n) {
+    for (uint32_t i = blockIdx.x * 256u + threadIdx.x; i < n; i += gridDim.x * 256u) dst[i] = src[i];
+}
+
+bool result_copy(const void* src, void* pinned, size_t bytes, hipStream_t s) {
+    const bool words = bytes % 4 == 0 && (uintptr_t)src % 4 == 0;
+    const uint32_t n = (uint32_t)(words ? bytes / 4 : bytes);
+    const dim3 grid(std::min<uint32_t>((n + 255) / 256, 256)), block(256);
+    if (words) hipLaunchKernelGGL(k_result<uint32_t>, grid, block, 0, s, (const uint32_t*)src, (uint32_t*)pinned, n);
+    else hipLaunchKernelGGL(k_result<uint8_t>, grid, block, 0, s, (const uint8_t*)src, (uint8_t*)pinned, n);
+    return check_launch("result copy");
+}
+}  // namespace
+
 // Resolves sm_capture_ws on the library's device (current during initialisation).
 void init_reduce_workspace() {
+    g_result_copy = result_copy;
     void* p = nullptr;
     if (check_hip(hipGetSymbolAddress(&p, HIP_SYMBOL(sm_capture_ws)), "hipGetSymbolAddress(sm_capture_ws)"))
         g_sm_capture_ws = (double*)p;

@@ -67,6 +67,10 @@ void init_reduce_workspace();
 bool launch_splitk_softmax(const float* part, int nsplit, int M, int N, double alpha, double beta, const float* c,
                            int cmode, float* Y, float* P, hipStream_t s);
 
+// Enqueues a copy of `bytes` from device memory to pinned host memory by a kernel; set by
+// init_reduce_workspace (runtime.hip holds no device code), null before.
+extern bool (*g_result_copy)(const void* src, void* pinned, size_t bytes, hipStream_t s);
+
 // ---- memory -----------------------------------------------------------------
 enum class Mem { kHostPinned, kHostMalloc, kDevOwned, kDevBorrowed, kHostForeign, kDevForeign };
 Mem classify(const void* p);     // registry first, then hipPointerGetAttributes

@@ -608,6 +608,8 @@ const double* device_cos_lut() { return lut_ready_on_device() ? S().d_lut : null
 
 using namespace tohip;
 
+bool (*tohip::g_result_copy)(const void*, void*, size_t, hipStream_t) = nullptr;
+
 // ======================= C ABI: lifecycle and extensions ==============================
 extern "C" {
 
@@ -721,12 +723,31 @@ static bool sync_copy_under_capture(const char* name) {
     return true;
 }
 
+// Small results: a kernel writes them to pinned host memory (its own launch, in stream
+// order), the stream is waited for and the bytes are copied on.  The runtime's copy to
+// pageable memory goes through its staging and a copy engine instead: 4 KB 24 -> 14.6 us,
+// and 88 us less per forward of the one-image residual network with its two outputs.
+// False: not taken (nothing enqueued).
+constexpr size_t kSmallResult = 256 << 10;
+
+static bool small_result(const Tensor* t, void* host_dst, size_t b, bool& ok) {
+    if (b > kSmallResult || !g_result_copy) return false;
+    void* pin = pinned_alloc(b);
+    if (!pin) return false;
+    ok = g_result_copy(t->data, pin, b, stream()) && check_hip(hipStreamSynchronize(stream()), "stream synchronize");
+    if (ok) memcpy(host_dst, pin, b);
+    pinned_free(pin);
+    return true;
+}
+
 int tensor_to_host(const Tensor* t, void* host_dst) {
     if (!tensor_sane(t, "tensor_to_host") || !host_dst) return -1;
     const size_t b = tensor_bytes(t);
     if (!b) return 0;
     if (is_dev(classify(t->data))) {
         if (sync_copy_under_capture("tensor_to_host")) return -1;
+        bool ok = false;
+        if (small_result(t, host_dst, b, ok)) return ok ? 0 : -1;
         if (!check_hip(hipMemcpyAsync(host_dst, t->data, b, hipMemcpyDeviceToHost, stream()), "D2H copy") ||
             !check_hip(hipStreamSynchronize(stream()), "stream synchronize"))
             return -1;

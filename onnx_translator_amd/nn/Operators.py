@@ -17,6 +17,7 @@ output formula of ``MaxPool.forward``.
 from __future__ import annotations
 
 import ctypes
+import functools
 
 import numpy as np
 
@@ -52,6 +53,17 @@ def _values(op, t):
 
 def _int_arr(vals):
     return (ctypes.c_int * len(vals))(*[int(v) for v in vals])
+
+
+@functools.lru_cache(maxsize=1024)
+def _conv_params(pads, strides, dilations, group):
+    """``ConvParams`` of these values (shared between equal ones: the library only reads
+    them; the struct keeps its arrays alive)."""
+    p = CConvParams()
+    p.pads, p.strides, p.dilations = [ctypes.cast(_int_arr(v), ctypes.POINTER(ctypes.c_int))
+                                      for v in (pads, strides, dilations)]
+    p.group = group
+    return p
 
 
 def _broadcast_dtype(a, b):
@@ -220,19 +232,14 @@ class Conv(Ops):
         self.lib.conv2d_forward.restype = None
 
     def _params(self):
-        keep = [_int_arr(self.pads), _int_arr(self.strides), _int_arr(self.dilations)]
-        p = CConvParams()
-        p.pads, p.strides, p.dilations = [ctypes.cast(k, ctypes.POINTER(ctypes.c_int)) for k in keep]
-        p.group = int(self.group)
-        return p, keep
+        return _conv_params(tuple(self.pads), tuple(self.strides), tuple(self.dilations), int(self.group))
 
     def forward(self, x: Tensor, w: Tensor, b: Tensor = None):
         N, _, H, W = x.size
         M, _, KH, KW = w.size
         OH, OW = _pool_out(H, W, self.pads, self.strides, self.dilations, KH, KW)
-        p, keep = self._params()
+        p = self._params()
         t = self._run("conv2d_forward", [x, w, b], (N, M, OH, OW), self.dtype, ctypes.byref(p))
-        del keep
         return _values(self, t)
 
     def forward_(self, x: Tensor_, w: Tensor_, b: Tensor_ = None):
@@ -258,13 +265,12 @@ class FusedConv(Conv):
         N, _, H, W = x.size
         M, _, KH, KW = w.size
         OH, OW = _pool_out(H, W, self.pads, self.strides, self.dilations, KH, KW)
-        p, keep = self._params()
+        p = self._params()
         relu = ctypes.c_int(self.relu)
 
         def arrange(ins, out):
             return (ins[0], ins[1], ins[2], ins[3], relu, out, ctypes.byref(p))
         t = self._run("conv2d_fused_forward", [x, w, b, skip], (N, M, OH, OW), self.dtype, arrange=arrange)
-        del keep
         return _values(self, t)
 
     def forward_(self, x: Tensor_, w: Tensor_, b: Tensor_ = None, skip: Tensor_ = None):
@@ -292,14 +298,13 @@ class FusedConvQDQ(FusedConv):
         N, _, H, W = x.size
         M, _, KH, KW = w.size
         OH, OW = _pool_out(H, W, self.pads, self.strides, self.dilations, KH, KW)
-        p, keep = self._params()
+        p = self._params()
         relu, code = ctypes.c_int(self.relu), ctypes.c_int(DTYPE_MAP[self.code_dtype])
 
         def arrange(ins, out):
             return (ins[0], ins[1], ins[2], ins[3], relu, ins[4], ins[5], ins[6], ins[7], code, out, ctypes.byref(p))
         t = self._run("conv2d_fused_qdq_forward", [x, w, b, skip, q_scale, q_zero_point, d_scale, d_zero_point],
                       (N, M, OH, OW), self.dtype, arrange=arrange)
-        del keep
         return _values(self, t)
 
     def forward_(self, x: Tensor_, w: Tensor_, b: Tensor_ = None, *rest):
@@ -325,14 +330,13 @@ class DequantizeConv(FusedConv):
         N, _, H, W = xq.size
         M, _, KH, KW = w.size
         OH, OW = _pool_out(H, W, self.pads, self.strides, self.dilations, KH, KW)
-        p, keep = self._params()
+        p = self._params()
         relu = ctypes.c_int(self.relu)
 
         def arrange(ins, out):
             return (ins[0], ins[1], ins[2], ins[3], ins[4], ins[5], relu, out, ctypes.byref(p))
         t = self._run("dequantize_conv2d_fused_forward", [xq, x_scale, x_zero_point, w, b, skip], (N, M, OH, OW),
                       self.dtype, arrange=arrange)
-        del keep
         return _values(self, t)
 
     def forward_(self, xq: Tensor_, x_scale: Tensor_ = None, x_zero_point: Tensor_ = None, w: Tensor_ = None,
@@ -408,10 +412,7 @@ class QConvBlock(Ops):
 
     def forward(self, x, x_scale, x_zero, w, w_sum, w_scale, bias=None, p=None, p_sum=None, p_scale=None,
                 skip=None, q_scale=None, q_zero=None):
-        keep = [_int_arr(self.pads), _int_arr(self.strides), _int_arr(self.dilations)]
-        prm = CConvParams()
-        prm.pads, prm.strides, prm.dilations = [ctypes.cast(k, ctypes.POINTER(ctypes.c_int)) for k in keep]
-        prm.group = 1
+        prm = _conv_params(tuple(self.pads), tuple(self.strides), tuple(self.dilations), 1)
         blk = CQConvBlock()
 
         def arrange(ins, out):
@@ -424,7 +425,6 @@ class QConvBlock(Ops):
         shape, dt = self._shape(x, w)
         t = self._run("qconv_block_forward", [x, x_scale, x_zero, w, w_sum, w_scale, bias, p, p_sum, p_scale, skip,
                                               q_scale, q_zero], shape, dt, arrange=arrange)
-        del keep
         return _values(self, t)
 
     def forward_(self, x, x_scale=None, x_zero=None, w=None, *rest):

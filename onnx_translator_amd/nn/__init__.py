@@ -21,6 +21,7 @@ Differences, all additive:
 from __future__ import annotations
 
 import ctypes
+import functools
 import os
 import threading
 
@@ -74,8 +75,14 @@ onnx_dtype_mapping = {
 PT = ctypes.POINTER(CTensor)
 
 
+@functools.lru_cache(maxsize=4096)
+def _shape_ints(shape):
+    return (ctypes.c_int * max(len(shape), 1))(*shape)
+
+
 def _shape_arr(shape):
-    return (ctypes.c_int * max(len(shape), 1))(*[int(s) for s in shape])
+    """C array of a shape (shared between equal shapes: the library only reads it)."""
+    return _shape_ints(tuple(map(int, shape)))
 
 
 class DeviceArray:
@@ -83,7 +90,7 @@ class DeviceArray:
 
     def __init__(self, lib, shape, dtype: str, ptr=None, zero: bool = True):
         self.lib = lib
-        self.shape = tuple(int(s) for s in shape)
+        self.shape = tuple(map(int, shape))
         self.dtype = dtype
         if ptr is None:
             shp = self.shape or (1,)

@@ -1246,7 +1246,7 @@ bool launch_conv_tiled_xq(const void* x, const void* w, const void* b, int dtb, 
         const double r = (double)t / (double)num_cus();
         return r / std::ceil(r);
     };
-    enum { kNone, kT64x128, kT128x128, kT64x256, kT128x256 };
+    enum { kNone, kT64x64, kT64x128, kT128x128, kT64x256, kT128x256 };
     const int khw = g.KH * g.KW;
     int plan = kNone;
     if (!direct && g.Cg % 16 == 0) {
@@ -1277,13 +1277,6 @@ bool launch_conv_tiled_xq(const void* x, const void* w, const void* b, int dtb, 
     auto blocks_of = [&](int p) {
         return tiles(p == kT128x128 || p == kT128x256 ? 128 : 64, p == kT64x128 || p == kT128x128 ? 128 : 256);
     };
-    // A few images: grids that leave CUs idle even with the k range split (slices 128
-    // deep, at most 8) take the smallest tiles and up to 16 slices of 64: one image of
-    // the residual network's blocks 2-4 29.4 / 30.0 / 30.4 -> 12.2 / 14.0 / 16.6 us, two of
-    // [512, 7, 7] 3x3 53 -> 23.5.
-    const int64_t coarse = std::min<int64_t>(g.Kg / 128, 8);
-    const bool tiny = !direct && plan != kNone && blocks_of(plan) * std::max<int64_t>(1, coarse) < num_cus();
-    if (tiny) plan = kT64x128;
     const int64_t blocks = blocks_of(plan);
     // Split-k slice count for grids smaller than the CU count: each slice
     // >= 128 deep, at most 8; the count whose block total balances best over
@@ -1293,7 +1286,7 @@ bool launch_conv_tiled_xq(const void* x, const void* w, const void* b, int dtb, 
     int split = 1;
     // (not under graph capture: the slices' workspace would have to outlive the call)
     if (blocks < num_cus() && !no_split && !stream_capturing(s)) {
-        const int smax = (int)(tiny ? std::min<int64_t>(g.Kg / 64, 16) : coarse);
+        const int smax = (int)std::min<int64_t>(g.Kg / 128, 8);
         const double base = balance(blocks);
         double best = base;
         for (int sp = 2; sp <= smax; sp++) {
@@ -1302,12 +1295,21 @@ bool launch_conv_tiled_xq(const void* x, const void* w, const void* b, int dtb, 
         }
         if (best < base * 1.05) split = 1;
     }
+    // A few images: where the plan leaves half of the CUs idle even so, 64x64 tiles (4 waves), with the
+    // slices as above.  The sums do not depend on the tiles, so this changes no bit (deeper
+    // splits, 16 slices of 64, were 10-20% faster still but move a quantized network's codes
+    // at other places).  One image of the residual network's blocks 2-4: 29.4 / 29.9 / 30.5
+    // -> 12.7 / 13.3 / 17.9 us, [2, 512, 7, 7] 3x3 53 -> 28.5.
+    if (!direct && plan != kNone && 2 * blocks * split <= num_cus()) plan = kT64x64;
     if (split > 1 && dty == kF32 && (!b || dtb == kF32) && yb * split < ((int64_t)1 << 31)) {
         // (an XQ launch always has an f32 output and an f32 or no bias)
         const float* bf = (const float*)b;
         float* yf = (float*)y;
         if (direct)
             return launch_conv_split_cfg<64, 256, 16, 2, 4, 1, XQ>(xf, wf, bf, yf, g, cg.group, ux, uw, split, epi, xq, s);
+        if (plan == kT64x64)
+            return launch_conv_split_cfg<64, 64, 16, 2, 2, 2, XQ, 2>(xf, wf, bf, yf, g, cg.group, ux, uw, split, epi, xq,
+                                                                     s);
         if (plan == kT64x128)
             return launch_conv_split_cfg<64, 128, 16, 2, 4, 2, XQ, 2>(xf, wf, bf, yf, g, cg.group, ux, uw, split, epi, xq,
                                                                       s);
@@ -1329,6 +1331,8 @@ bool launch_conv_tiled_xq(const void* x, const void* w, const void* b, int dtb, 
         launch_conv_tiled_cfg<64, 256, 8, 2, 4, 1, XQ>(xf, wf, b, dtb, y, dty, g, cg.group, ux, uw, uy, epi, xq, s);
     else if (direct)
         launch_conv_tiled_cfg<64, 256, 16, 2, 4, 1, XQ>(xf, wf, b, dtb, y, dty, g, cg.group, ux, uw, uy, epi, xq, s);
+    else if (plan == kT64x64)
+        launch_conv_tiled_cfg<64, 64, 16, 2, 2, 2, XQ, 2>(xf, wf, b, dtb, y, dty, g, cg.group, ux, uw, uy, epi, xq, s);
     else if (plan == kT64x128)
         launch_conv_tiled_cfg<64, 128, 16, 2, 4, 2, XQ, 2>(xf, wf, b, dtb, y, dty, g, cg.group, ux, uw, uy, epi, xq, s);
     else if (plan == kT128x128)

@@ -1,4 +1,4 @@
-"""f32 convolutions of a few images (64x128 tiles with up to 16 slices of k) against the
+"""f32 convolutions of a few images (64x64 tiles, with and without slices of k) against the
 oracle (tensor_ops.c:1036-1114), plain and with the fused epilogue, whose bits are the
 separate calls'; tolerance assert_close's 1e-5 for f32 sums."""
 import numpy as np

@@ -57,4 +57,19 @@ bool conv_depthwise_shape(const ConvGeom& g);
 bool launch_conv_f16(const void* x, const void* w, const void* b, int dtb, void* y, int dty, const ConvGeom& g,
                      hipStream_t s);
 
+// A Gemm of halves in the layouts and sizes that gemm.hip's f16 kernels do not fetch
+// directly (convh.hip): c f32, cmode 0 none, 1 one value, 2 per column, 3 per row.
+// 0: not taken; 1: done; -1: error set; 2: *nsplit slices of M x N f32 sums at *part, which
+// the caller reduces (with the epilogue) and then frees *ws.
+struct GemmH {
+    const void* A;
+    const void* B;
+    void* Y;
+    int ta, tb, dty, M, N, K;
+    double alpha, beta;
+    const float* c;
+    int cmode;
+};
+int launch_gemm_f16_packed(const GemmH& q, hipStream_t s, float** part, int* nsplit, void** ws);
+
 }  // namespace tohip

@@ -126,6 +126,24 @@ __device__ __forceinline__ void load_lds16(__amdgpu_buffer_rsrc_t r, _Float16* t
     __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)to, 16, off, 0, 0, 0);
 }
 
+// What is added to a sum: a convolution's bias (one value per channel), or a Gemm's
+// alpha * acc + beta * c in double, rounded once (c f32: cmode 0 none, 1 one
+// value, 2 per column, 3 per row).
+struct EpiH {
+    const void* b;
+    int dtb;
+    int cmode;
+    double alpha, beta;
+    __device__ __forceinline__ float bias(int m) const {
+        return b ? (dtb == kF16 ? (float)((const _Float16*)b)[m] : ((const float*)b)[m]) : 0.0f;
+    }
+    __device__ __forceinline__ float gemm(float acc, int m, int n) const {
+        double r = alpha * (double)acc;
+        if (cmode) r += beta * (double)((const float*)b)[cmode == 1 ? 0 : cmode == 2 ? n : m];
+        return (float)r;
+    }
+};
+
 // Waits until at most N of this wave's memory loads are outstanding (they complete in
 // order; N <= 63) and its LDS reads have returned (the barrier after it tells the other
 // waves that a slot may be filled again).
@@ -143,10 +161,9 @@ template <int N> __device__ __forceinline__ void wait_loads() {
 // the tap, the channel chunk and their offset are worked out once per k-tile and lane.
 // Padding taps, rows past M and chunks past KC lie past the buffer's range: zeros.
 // SPLIT: slice z covers k-tiles [z * kt_per, ...) and stores f32 sums to Y + z * total.
-template <int BM, int BP, int R, int ODT, bool SPLIT>
+template <int BM, int BP, int R, int ODT, bool SPLIT, bool GEMM>
 __global__ __launch_bounds__(kHThreads, 2) void k_convh(const uint4* __restrict__ Xp, const uint4* __restrict__ Wp,
-                                                     const void* __restrict__ Bv, int dtb, void* __restrict__ Y, ConvH g,
-                                                     int ntm, int ntp, int kt_per, int64_t total, int ywidth) {
+                                                     EpiH epi, void* __restrict__ Y, ConvH g, int ntm, int ntp, int kt_per, int64_t total, int ywidth) {
     constexpr int TI = BM / 64, TJ = BP / 64, NA = BM / 32, NB = BP / 32;
     // the ring's slots: distinct arrays, so that a read of one does not wait for the
     // loads in flight to the others
@@ -261,9 +278,6 @@ __global__ __launch_bounds__(kHThreads, 2) void k_convh(const uint4* __restrict_
         }
     }
     wait_loads<0>();        // nothing may land in LDS after the block ends or reuses it
-    auto bias_of = [&](int m) {
-        return Bv ? (dtb == kF16 ? (float)((const _Float16*)Bv)[m] : ((const float*)Bv)[m]) : 0.0f;
-    };
     if constexpr (ODT == kF16 && !SPLIT) {
         // Halves leave through LDS, V pixels (V the power of two up to 8 that divides
         // OHW, so they share an image and an aligned address) of one channel per thread
@@ -276,10 +290,14 @@ __global__ __launch_bounds__(kHThreads, 2) void k_convh(const uint4* __restrict_
 #pragma unroll
             for (int r = 0; r < 16; r++) {
                 const int row = wm * (BM / 2) + i * 32 + 8 * (r >> 2) + 4 * h + (r & 3);
-                const float bias = m0 + row < g.Mg ? bias_of(grp * g.Mg + m0 + row) : 0.0f;
+                const int m = grp * g.Mg + min(m0 + row, g.Mg - 1);
+                const float bias = GEMM ? 0.0f : epi.bias(m);
 #pragma unroll
-                for (int j = 0; j < TJ; j++)
-                    out[row * BP + wn * (BP / 2) + j * 32 + lr] = enc_f16(acc[i][j][r] + bias);
+                for (int j = 0; j < TJ; j++) {
+                    const int c = wn * (BP / 2) + j * 32 + lr;
+                    const float v = GEMM ? epi.gemm(acc[i][j][r], m, min(p0 + c, g.P - 1)) : acc[i][j][r] + bias;
+                    out[row * BP + c] = enc_f16(v);
+                }
             }
         __syncthreads();
         auto store = [&](auto tag) {
@@ -312,7 +330,7 @@ __global__ __launch_bounds__(kHThreads, 2) void k_convh(const uint4* __restrict_
                 const int m = grp * g.Mg + ml;
                 const int64_t yi = ((int64_t)n * g.M + m) * g.OHW + r0;
                 if constexpr (SPLIT) ((gfloat*)Y)[(int64_t)blockIdx.z * total + yi] = acc[i][j][r];
-                else ((gfloat*)Y)[yi] = acc[i][j][r] + bias_of(m);
+                else ((gfloat*)Y)[yi] = GEMM ? epi.gemm(acc[i][j][r], m, p) : acc[i][j][r] + epi.bias(m);
             }
     }
 }
@@ -333,8 +351,8 @@ __global__ __launch_bounds__(256) void k_convh_reduce(const float* __restrict__ 
     st_d<ODT>(Y, i, acc);
 }
 
-template <int BM, int BP, int R>
-void launch_tiles(const uint4* xp, const uint4* wp, const void* b, int dtb, void* y, int dty, float* part,
+template <int BM, int BP, int R, bool GEMM>
+void launch_tiles(const uint4* xp, const uint4* wp, const EpiH& epi, void* y, int dty, float* part,
                   const ConvH& g, int split, int64_t total, hipStream_t s) {
     const int ntm = (g.Mg + BM - 1) / BM, ntp = (g.P + BP - 1) / BP, nk = (g.KC + 7) / 8;
     const int kt_per = (nk + split - 1) / split;
@@ -342,17 +360,15 @@ void launch_tiles(const uint4* xp, const uint4* wp, const void* b, int dtb, void
     while (yw > 1 && (g.OHW % yw || (uintptr_t)y % (2 * yw))) yw /= 2;
     const dim3 grid((unsigned)(ntm * ntp), (unsigned)g.group, (unsigned)split), blk(kHThreads);
     if (split > 1)
-        hipLaunchKernelGGL((k_convh<BM, BP, R, kF32, true>), grid, blk, 0, s, xp, wp, b, dtb, (void*)part, g, ntm, ntp,
+        hipLaunchKernelGGL((k_convh<BM, BP, R, kF32, true, false>), grid, blk, 0, s, xp, wp, epi, (void*)part, g, ntm, ntp,
                            kt_per, total, yw);
     else if (dty == kF16)
-        hipLaunchKernelGGL((k_convh<BM, BP, R, kF16, false>), grid, blk, 0, s, xp, wp, b, dtb, y, g, ntm, ntp, kt_per,
+        hipLaunchKernelGGL((k_convh<BM, BP, R, kF16, false, GEMM>), grid, blk, 0, s, xp, wp, epi, y, g, ntm, ntp, kt_per,
                            total, yw);
     else
-        hipLaunchKernelGGL((k_convh<BM, BP, R, kF32, false>), grid, blk, 0, s, xp, wp, b, dtb, y, g, ntm, ntp, kt_per,
+        hipLaunchKernelGGL((k_convh<BM, BP, R, kF32, false, GEMM>), grid, blk, 0, s, xp, wp, epi, y, g, ntm, ntp, kt_per,
                            total, yw);
 }
-
-}  // namespace
 
 // Ring slots per tile shape: more loads in flight against more blocks per CU.  128x128
 // with three or four slots (one block per CU) takes [32, 64, 56, 56] -> 256 1x1 from 46.5
@@ -360,6 +376,38 @@ void launch_tiles(const uint4* xp, const uint4* wp, const void* b, int dtb, void
 // 31.7 against 26.0 us at [32, 128, 28, 28] 3x3 (its LDS reads, two per MFMA, need the
 // blocks more than the prefetch).
 constexpr int kRing128x128 = 2, kRing64x128 = 3, kRing64x64 = 2;
+
+// Tile shape and k slices of a GEMM of Mg rows per group, P columns and KC chunks of k.
+struct TilesH {
+    int bm, bp, split;
+};
+
+TilesH tiles_h(int64_t P, int64_t Mg, int64_t group, int64_t KC) {
+    // Tiles: 128x128 from two blocks per CU on ([32, 128, 28, 28] 3x3, 196 of them: 40
+    // against 24.6 us with 392 of 64x128), 64x128 from one and a half on, else 64x64; then,
+    // with less than one block per CU, slices of k (each at least four k-tiles deep).
+    const int cus = num_cus();
+    auto tiles = [&](int bm, int bp) { return ((P + bp - 1) / bp) * ((Mg + bm - 1) / bm) * group; };
+    int bm = Mg > 64 ? 128 : 64, bp = 128;
+    if (bm == 128 && tiles(128, 128) < 2 * cus) bm = 64;
+    if (2 * tiles(bm, bp) < 3 * cus) bp = 64;
+    const int nk = (int)((KC + 7) / 8);
+    int split = 1;
+    const int64_t nt = tiles(bm, bp);
+    if (nt < cus) split = (int)std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>((2 * cus + nt - 1) / nt, 16), nk / 4));
+    if (split > 1) split = (nk + (nk + split - 1) / split - 1) / ((nk + split - 1) / split);     // no empty slice
+    return TilesH{bm, bp, split};
+}
+
+template <bool GEMM>
+void launch_tiles_h(const TilesH& t, const uint4* xp, const uint4* wp, const EpiH& epi, void* y, int dty, float* part,
+                   const ConvH& g, int64_t total, hipStream_t s) {
+    if (t.bm == 128) launch_tiles<128, 128, kRing128x128, GEMM>(xp, wp, epi, y, dty, part, g, t.split, total, s);
+    else if (t.bp == 128) launch_tiles<64, 128, kRing64x128, GEMM>(xp, wp, epi, y, dty, part, g, t.split, total, s);
+    else launch_tiles<64, 64, kRing64x64, GEMM>(xp, wp, epi, y, dty, part, g, t.split, total, s);
+}
+
+}  // namespace
 
 bool launch_conv_f16(const void* x, const void* w, const void* b, int dtb, void* y, int dty, const ConvGeom& cg,
                      hipStream_t s) {
@@ -388,20 +436,9 @@ bool launch_conv_f16(const void* x, const void* w, const void* b, int dtb, void*
     g.fd_c8 = make_fastdiv((uint32_t)C8);
     g.fd_kw = make_fastdiv((uint32_t)g.KW);
     g.fd_khw = make_fastdiv((uint32_t)KHW);
-    // Tiles: 128x128 from two blocks per CU on ([32, 128, 28, 28] 3x3, 196 of them: 40
-    // against 24.6 us with 392 of 64x128), 64x128 from one and a half on, else 64x64; then,
-    // with less than one block per CU, slices of k (each at least four k-tiles deep).
-    const int cus = num_cus();
-    auto tiles = [&](int bm, int bp) { return ((P + bp - 1) / bp) * ((cg.Mg + bm - 1) / bm) * cg.group; };
-    int bm = cg.Mg > 64 ? 128 : 64, bp = 128;
-    if (bm == 128 && tiles(128, 128) < 2 * cus) bm = 64;
-    if (2 * tiles(bm, bp) < 3 * cus) bp = 64;
-    const int nk = (int)((KC + 7) / 8);
-    int split = 1;
-    const int64_t nt = tiles(bm, bp);
-    if (nt < cus) split = (int)std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>((2 * cus + nt - 1) / nt, 16), nk / 4));
-    if (split > 1) split = (nk + (nk + split - 1) / split - 1) / ((nk + split - 1) / split);     // no empty slice
+    const TilesH t = tiles_h(P, cg.Mg, cg.group, KC);
     auto up = [](int64_t v) { return (v + 255) / 256 * 256; };
+    const int split = t.split;
     const int64_t pb = split > 1 ? (int64_t)split * total * 4 : 0;
     char* ws = (char*)pool_alloc((size_t)(up(xb) + up(wb) + pb));
     if (!ws) return false;
@@ -416,9 +453,7 @@ bool launch_conv_f16(const void* x, const void* w, const void* b, int dtb, void*
     else
         hipLaunchKernelGGL(k_convh_pack<false>, pg, pblk, 0, s, (const uint16_t*)x, (const uint16_t*)w, xp, wp, g,
                            (int)xblocks, qblocks);
-    if (bm == 128) launch_tiles<128, 128, kRing128x128>(xp, wp, b, dtb, y, dty, part, g, split, total, s);
-    else if (bp == 128) launch_tiles<64, 128, kRing64x128>(xp, wp, b, dtb, y, dty, part, g, split, total, s);
-    else launch_tiles<64, 64, kRing64x64>(xp, wp, b, dtb, y, dty, part, g, split, total, s);
+    launch_tiles_h<false>(t, xp, wp, EpiH{b, dtb, 0, 0.0, 0.0}, y, dty, part, g, total, s);
     if (split > 1) {
         const dim3 rg((unsigned)((total + 255) / 256));
         const FastDiv fo = g.fd_ohw, fm = make_fastdiv((uint32_t)g.M);
@@ -427,6 +462,71 @@ bool launch_conv_f16(const void* x, const void* w, const void* b, int dtb, void*
     }
     pool_free(ws);   // stream-ordered reuse: later work on this stream runs after the kernels
     return true;
+}
+
+// Y[M, N] = alpha A' B' + beta C of halves as the GEMM above: A's rows are the output
+// channels, B's columns the pixels of one image, K the channels.  Each operand is copied
+// into rows of chunks first: one stored with k along its rows (A [M, K], B [N, K]) by the
+// weights' part of k_convh_pack, one stored the other way by the images' part.  Against the
+// 128x128x32 kernel without a k split that took these layouts: [512, 1024] x [1024, 4096]
+// 85 -> 26 us, [87, 1728] x [1728, 421] 177 -> 17.6, [300, 1003] x [1001, 1003]^T 93 -> 18;
+// short k is left to it, as three launches cost 12.5 us ([20, 80] x [80, 64] 12.0, [7, 65] x
+// [64, 65]^T 9.0).
+constexpr int kGemmHMinK = 128;
+
+int launch_gemm_f16_packed(const GemmH& q, hipStream_t s, float** part, int* nsplit, void** ws) {
+    if ((q.dty != kF16 && q.dty != kF32) || q.M < 1 || q.N < 1 || q.K < kGemmHMinK || stream_capturing(s)) return 0;
+    const int64_t KC = ((int64_t)q.K + 7) / 8, reach = (int64_t)1 << 31;
+    const int64_t ab = (int64_t)q.M * KC * 16, bb = (int64_t)q.N * KC * 16, total = (int64_t)q.M * q.N;
+    if (ab >= reach || bb >= reach || total >= reach / 4) return 0;
+    auto up = [](int64_t v) { return (v + 255) / 256 * 256; };
+    const TilesH t = tiles_h(q.N, q.M, 1, KC);
+    const int64_t pb = t.split > 1 ? (int64_t)t.split * total * 4 : 0;
+    char* w = (char*)pool_alloc((size_t)(up(ab) + up(bb) + pb));
+    if (!w) return -1;
+    uint4 *ap = (uint4*)w, *bp = (uint4*)(w + up(ab));
+    ConvH g;
+    g.H = 1; g.KW = 1; g.pt = g.pl = 0; g.sh = g.sw = g.dh = g.dw = 1; g.group = 1;
+    g.C = g.Cg = q.K; g.KHW = 1; g.C8 = g.KC = (int)KC;
+    g.rb = (uint32_t)(KC * 16);
+    g.fd_c8 = make_fastdiv((uint32_t)KC);
+    g.fd_kw = g.fd_khw = make_fastdiv(1);
+    // n rows of chunks from src into dst; along: k runs along src's rows
+    auto pack = [&](const void* src, int n, bool along, uint4* dst) {
+        g.HW = g.NHW = g.M = n;
+        g.fd_hw = make_fastdiv((uint32_t)n);
+        const int qblocks = (int)((KC + 7) / 8);
+        const uint16_t* h = (const uint16_t*)src;
+        const dim3 blk(kHThreads);
+        if (along) {
+            const dim3 grid((unsigned)(((int64_t)n * KC + kHThreads - 1) / kHThreads));
+            hipLaunchKernelGGL(k_convh_pack<false>, grid, blk, 0, s, h, h, dst, dst, g, 0, qblocks);
+        } else {
+            const int xblocks = (n + 63) / 64 * qblocks;
+            if (n % 2 == 0 && ((uintptr_t)src & 3) == 0)
+                hipLaunchKernelGGL(k_convh_pack<true>, dim3((unsigned)xblocks), blk, 0, s, h, h, dst, dst, g, xblocks, qblocks);
+            else
+                hipLaunchKernelGGL(k_convh_pack<false>, dim3((unsigned)xblocks), blk, 0, s, h, h, dst, dst, g, xblocks, qblocks);
+        }
+    };
+    pack(q.A, q.M, !q.ta, ap);
+    pack(q.B, q.N, q.tb != 0, bp);
+    g.W = g.OW = g.OHW = g.P = g.HW = g.NHW = q.N;
+    g.M = g.Mg = q.M;
+    g.xbytes = (uint32_t)bb; g.wbytes = (uint32_t)ab;
+    g.fd_hw = g.fd_ohw = g.fd_ow = make_fastdiv((uint32_t)q.N);
+    const EpiH epi{q.c, kF32, q.c ? q.cmode : 0, q.alpha, q.beta};
+    float* ps = (float*)(w + up(ab) + up(bb));
+    launch_tiles_h<true>(t, bp, ap, epi, q.Y, q.dty, ps, g, total, s);
+    if (t.split == 1) {
+        pool_free(w);    // stream-ordered reuse
+        return 1;
+    }
+    const int nk = (int)((KC + 7) / 8), per = (nk + t.split - 1) / t.split;
+    *part = ps;
+    *nsplit = (nk + per - 1) / per;
+    *ws = w;
+    return 2;
 }
 
 }  // namespace tohip

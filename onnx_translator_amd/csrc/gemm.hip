@@ -20,13 +20,17 @@
 //    small grids.
 //  * k_gemm_rows — the same operands with at most 64 rows of A and B [N, K]: one
 //    pass over B straight into the MFMA operands.
-//  * k_gemm_mfma_f16 — the other f16 transposes: 128x128x32 tiles.
+//  * convh.hip's f16 GEMM — the other f16 layouts and sizes, through copies of the
+//    operands in rows of 16-byte chunks.
+//  * k_gemm_mfma_f16 — those under graph capture (no workspace) or with a bias of
+//    another type: 128x128x32 tiles.
 //  * k_gemm_exact — fp64, sequential k, no contraction: bit-identical to the
 //    reference for every dtype combination.  Used for f64 / int32 / int64
 //    operands and when exact mode is on.
 // The epilogue is shared: alpha * acc + beta * bias in double, then st_d.
 #include <algorithm>
 
+#include "conv.h"
 #include "runtime.h"
 
 namespace tohip {
@@ -1351,7 +1355,27 @@ void gemm_impl(const char* name, const Tensor* A, const Tensor* B, const Tensor*
                 const dim3 grid((N + kBN - 1) / kBN, (M + kBM - 1) / kBM);
                 const int vec = ((g.lda % 8) == 0 && (g.ldb % 8) == 0 && ((uintptr_t)g.A & 15) == 0 &&
                                  ((uintptr_t)g.B & 15) == 0) ? 1 : 0;
-                if (!transA && transB && vec && launch_f16_nt(g, s)) {
+                int packed = 0;
+                if (!(!transA && transB && vec) && (has_c ? g.c.dt == kF32 && g.c.mode <= 3 : true)) {
+                    float* part = nullptr;
+                    int nsplit = 0;
+                    void* ws = nullptr;
+                    const GemmH q{g.A, g.B, g.Y, transA, transB, g.dty, M, N, K, g.alpha, g.beta, (const float*)g.c.p,
+                                  g.c.mode};
+                    packed = launch_gemm_f16_packed(q, s, &part, &nsplit, &ws);
+                    if (packed < 0) { st.finish(); return; }
+                    if (packed == 2) {
+                        const dim3 rgrid((unsigned)(((int64_t)M * N + 255) / 256));
+                        const FastDiv fd_n = make_fastdiv((uint32_t)N);
+                        if (g.dty == kF16)
+                            hipLaunchKernelGGL((k_splitk_reduce<kF16>), rgrid, dim3(256), 0, s, g, (const float*)part, nsplit, fd_n);
+                        else
+                            hipLaunchKernelGGL((k_splitk_reduce<kF32>), rgrid, dim3(256), 0, s, g, (const float*)part, nsplit, fd_n);
+                        pool_free(ws);
+                    }
+                }
+                if (packed) {
+                } else if (!transA && transB && vec && launch_f16_nt(g, s)) {
                 } else if (!transA && transB) launch_f16_y<false, true>(g, grid, vec, s);
                 else if (!transA && !transB) launch_f16_y<false, false>(g, grid, vec, s);
                 else if (transA && transB) launch_f16_y<true, true>(g, grid, vec, s);

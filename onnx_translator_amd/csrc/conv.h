@@ -59,8 +59,8 @@ bool launch_conv_f16(const void* x, const void* w, const void* b, int dtb, void*
 
 // A Gemm of halves in the layouts and sizes that gemm.hip's f16 kernels do not fetch
 // directly (convh.hip): c f32, cmode 0 none, 1 one value, 2 per column, 3 per row.
-// 0: not taken; 1: done; -1: error set; 2: *nsplit slices of M x N f32 sums at *part, which
-// the caller reduces (with the epilogue) and then frees *ws.
+// 0: not taken (no memory for the copies included); 1: done; 2: *nsplit slices of M x N
+// f32 sums at *part, which the caller reduces (with the epilogue) and then frees *ws.
 struct GemmH {
     const void* A;
     const void* B;

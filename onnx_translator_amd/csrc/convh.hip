@@ -440,7 +440,7 @@ bool launch_conv_f16(const void* x, const void* w, const void* b, int dtb, void*
     auto up = [](int64_t v) { return (v + 255) / 256 * 256; };
     const int split = t.split;
     const int64_t pb = split > 1 ? (int64_t)split * total * 4 : 0;
-    char* ws = (char*)pool_alloc((size_t)(up(xb) + up(wb) + pb));
+    char* ws = (char*)pool_alloc((size_t)(up(xb) + up(wb) + pb), true);
     if (!ws) return false;
     uint4 *xp = (uint4*)ws, *wp = (uint4*)(ws + up(xb));
     float* part = (float*)(ws + up(xb) + up(wb));
@@ -482,8 +482,8 @@ int launch_gemm_f16_packed(const GemmH& q, hipStream_t s, float** part, int* nsp
     auto up = [](int64_t v) { return (v + 255) / 256 * 256; };
     const TilesH t = tiles_h(q.N, q.M, 1, KC);
     const int64_t pb = t.split > 1 ? (int64_t)t.split * total * 4 : 0;
-    char* w = (char*)pool_alloc((size_t)(up(ab) + up(bb) + pb));
-    if (!w) return -1;
+    char* w = (char*)pool_alloc((size_t)(up(ab) + up(bb) + pb), true);
+    if (!w) return 0;
     uint4 *ap = (uint4*)w, *bp = (uint4*)(w + up(ab));
     ConvH g;
     g.H = 1; g.KW = 1; g.pt = g.pl = 0; g.sh = g.sw = g.dh = g.dw = 1; g.group = 1;

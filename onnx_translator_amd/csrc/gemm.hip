@@ -1177,7 +1177,7 @@ bool launch_f16_nt(const GemmArgs& g, hipStream_t s) {
 // fused weight-only-quantized Gemm and the unfused DequantizeLinear -> Gemm
 // pair run the same schedule and return the same bits.
 // Returns 1 when launched, 0 when the operands do not fit the kernel (caller
-// falls back), -1 on an allocation failure (error set).
+// falls back).
 int nt_split_plan(int M, int N, int K, bool& big) {
     const int64_t big_tiles = (int64_t)((M + 127) / 128) * ((N + 255) / 256);
     big = big_tiles >= 192;
@@ -1253,15 +1253,14 @@ int launch_f32_nt(const GemmArgs& g, const WoqB& q, hipStream_t s, float* probs 
         launch_nt_kernel<128, 256, 16, 2, 4, BQ, false, KN>(g, q, 0, 1, ydt, s);
         return 1;
     }
-    if (split <= 1) {
+    const int kchunk = ((g.K + split - 1) / std::max(split, 1) + 15) / 16 * 16;
+    const int nsplit = split > 1 ? (g.K + kchunk - 1) / kchunk : 1;
+    const int64_t mn = (int64_t)g.M * g.N;
+    float* part = split > 1 ? (float*)pool_alloc((size_t)nsplit * mn * sizeof(float), true) : nullptr;
+    if (!part) {    // one slice, or no memory for several
         launch_nt_kernel<128, 64, 16, 2, 2, BQ, false, KN>(g, q, 0, 1, ydt, s);
         return 1;
     }
-    const int kchunk = ((g.K + split - 1) / split + 15) / 16 * 16;
-    const int nsplit = (g.K + kchunk - 1) / kchunk;
-    const int64_t mn = (int64_t)g.M * g.N;
-    float* part = (float*)pool_alloc((size_t)nsplit * mn * sizeof(float));
-    if (!part) return -1;
     GemmArgs gp = g;
     gp.Y = part;
     launch_nt_kernel<128, 64, 16, 2, 2, BQ, true, KN>(gp, q, kchunk, nsplit, kF32, s);
@@ -1363,7 +1362,6 @@ void gemm_impl(const char* name, const Tensor* A, const Tensor* B, const Tensor*
                     const GemmH q{g.A, g.B, g.Y, transA, transB, g.dty, M, N, K, g.alpha, g.beta, (const float*)g.c.p,
                                   g.c.mode};
                     packed = launch_gemm_f16_packed(q, s, &part, &nsplit, &ws);
-                    if (packed < 0) { st.finish(); return; }
                     if (packed == 2) {
                         const dim3 rgrid((unsigned)(((int64_t)M * N + 255) / 256));
                         const FastDiv fd_n = make_fastdiv((uint32_t)N);
@@ -1386,7 +1384,6 @@ void gemm_impl(const char* name, const Tensor* A, const Tensor* B, const Tensor*
                                    ((uintptr_t)g.B & 3) == 0;
                 const WoqB f32_b{nullptr, nullptr, 0, 0};
                 const int r = !tiled ? 0 : transB ? launch_f32_nt<0>(g, f32_b, s, probs) : launch_f32_nt<0, true>(g, f32_b, s, probs);
-                if (r < 0) { st.finish(); return; }
                 if (r == 2 && softmax_done) *softmax_done = true;
                 done = r >= 1 || launch_f32_mfma(g, dta, dtb, transA, transB, s);
             }

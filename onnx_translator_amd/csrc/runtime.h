@@ -80,8 +80,9 @@ inline bool is_dev(Mem m) { return m == Mem::kDevOwned || m == Mem::kDevBorrowed
 // released on.  Refused (nullptr, error set) while the library stream is being
 // captured into a graph: a buffer taken inside a capture goes back to the pool
 // when the call returns while the graph goes on using it, and a fresh one would
-// need hipMalloc inside the capture.
-void* pool_alloc(size_t bytes);
+// need hipMalloc inside the capture.  quiet: no error is set, for a caller that has a
+// path without the memory.
+void* pool_alloc(size_t bytes, bool quiet = false);
 void pool_free(void* p);
 
 size_t tensor_bytes(const Tensor* t);

@@ -310,10 +310,10 @@ static void* take_cached(std::multimap<size_t, void*>& fl, size_t need, size_t& 
     return p;
 }
 
-void* pool_alloc(size_t bytes) {
+void* pool_alloc(size_t bytes, bool quiet) {
     State& s = S();
     if (stream_capturing(stream())) {
-        set_error("device memory requested while the library stream is being captured into a graph "
+        if (!quiet) set_error("device memory requested while the library stream is being captured into a graph "
                   "(allocate before the capture; captured calls must not allocate)");
         return nullptr;
     }
@@ -349,7 +349,7 @@ void* pool_alloc(size_t bytes) {
         s.dev_cached = 0;
         if (hipMalloc(&p, need) != hipSuccess) {
             (void)hipGetLastError();
-            set_error("hipMalloc(%zu) failed: out of device memory", need);
+            if (!quiet) set_error("hipMalloc(%zu) failed: out of device memory", need);
             return nullptr;
         }
     }

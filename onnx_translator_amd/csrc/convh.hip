@@ -465,11 +465,12 @@ bool launch_conv_f16(const void* x, const void* w, const void* b, int dtb, void*
 }
 
 // Y[M, N] = alpha A' B' + beta C of halves as the GEMM above: A's rows are the output
-// channels, B's columns the pixels of one image, K the channels.  Each operand is copied
-// into rows of chunks first: one stored with k along its rows (A [M, K], B [N, K]) by the
-// weights' part of k_convh_pack, one stored the other way by the images' part.  Against the
+// channels, B's columns the pixels of one image, K the channels.  An operand with k along its
+// rows (A [M, K], B [N, K]) in whole, aligned chunks is read where it lies; any other is
+// copied into rows of chunks first, by the weights' part of k_convh_pack where k runs along
+// its rows, else by the images' part.  Against the
 // 128x128x32 kernel without a k split that took these layouts: [512, 1024] x [1024, 4096]
-// 85 -> 26 us, [87, 1728] x [1728, 421] 177 -> 17.6, [300, 1003] x [1001, 1003]^T 93 -> 18;
+// 85 -> 23 us, [87, 1728] x [1728, 421] 177 -> 17.6, [300, 1003] x [1001, 1003]^T 93 -> 18;
 // short k is left to it, as three launches cost 12.5 us ([20, 80] x [80, 64] 12.0, [7, 65] x
 // [64, 65]^T 9.0).
 constexpr int kGemmHMinK = 128;
@@ -482,9 +483,13 @@ int launch_gemm_f16_packed(const GemmH& q, hipStream_t s, float** part, int* nsp
     auto up = [](int64_t v) { return (v + 255) / 256 * 256; };
     const TilesH t = tiles_h(q.N, q.M, 1, KC);
     const int64_t pb = t.split > 1 ? (int64_t)t.split * total * 4 : 0;
-    char* w = (char*)pool_alloc((size_t)(up(ab) + up(bb) + pb), true);
-    if (!w) return 0;
-    uint4 *ap = (uint4*)w, *bp = (uint4*)(w + up(ab));
+    // k along the rows, whole chunks and an aligned base: the operand is its own copy
+    const bool a_own = !q.ta && q.K % 8 == 0 && ((uintptr_t)q.A & 15) == 0;
+    const bool b_own = q.tb && q.K % 8 == 0 && ((uintptr_t)q.B & 15) == 0;
+    const int64_t ac = a_own ? 0 : up(ab), bc = b_own ? 0 : up(bb);
+    char* w = nullptr;
+    if (ac + bc + pb && !(w = (char*)pool_alloc((size_t)(ac + bc + pb), true))) return 0;
+    const uint4 *ap = a_own ? (const uint4*)q.A : (const uint4*)w, *bp = b_own ? (const uint4*)q.B : (const uint4*)(w + ac);
     ConvH g;
     g.H = 1; g.KW = 1; g.pt = g.pl = 0; g.sh = g.sw = g.dh = g.dw = 1; g.group = 1;
     g.C = g.Cg = q.K; g.KHW = 1; g.C8 = g.KC = (int)KC;
@@ -509,17 +514,17 @@ int launch_gemm_f16_packed(const GemmH& q, hipStream_t s, float** part, int* nsp
                 hipLaunchKernelGGL(k_convh_pack<false>, dim3((unsigned)xblocks), blk, 0, s, h, h, dst, dst, g, xblocks, qblocks);
         }
     };
-    pack(q.A, q.M, !q.ta, ap);
-    pack(q.B, q.N, q.tb != 0, bp);
+    if (!a_own) pack(q.A, q.M, !q.ta, (uint4*)w);
+    if (!b_own) pack(q.B, q.N, q.tb != 0, (uint4*)(w + ac));
     g.W = g.OW = g.OHW = g.P = g.HW = g.NHW = q.N;
     g.M = g.Mg = q.M;
     g.xbytes = (uint32_t)bb; g.wbytes = (uint32_t)ab;
     g.fd_hw = g.fd_ohw = g.fd_ow = make_fastdiv((uint32_t)q.N);
     const EpiH epi{q.c, kF32, q.c ? q.cmode : 0, q.alpha, q.beta};
-    float* ps = (float*)(w + up(ab) + up(bb));
+    float* ps = t.split > 1 ? (float*)(w + ac + bc) : nullptr;
     launch_tiles_h<true>(t, bp, ap, epi, q.Y, q.dty, ps, g, total, s);
     if (t.split == 1) {
-        pool_free(w);    // stream-ordered reuse
+        if (w) pool_free(w);    // stream-ordered reuse
         return 1;
     }
     const int nk = (int)((KC + 7) / 8), per = (nk + t.split - 1) / t.split;

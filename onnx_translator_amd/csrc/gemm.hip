@@ -20,8 +20,8 @@
 //    small grids.
 //  * k_gemm_rows — the same operands with at most 64 rows of A and B [N, K]: one
 //    pass over B straight into the MFMA operands.
-//  * convh.hip's f16 GEMM — the other f16 layouts and sizes, through copies of the
-//    operands in rows of 16-byte chunks.
+//  * convh.hip's f16 GEMM — small f16 grids, and the other f16 layouts and sizes through
+//    copies of the operands in rows of 16-byte chunks.
 //  * k_gemm_mfma_f16 — those under graph capture (no workspace) or with a bias of
 //    another type: 128x128x32 tiles.
 //  * k_gemm_exact — fp64, sequential k, no contraction: bit-identical to the
@@ -1154,6 +1154,16 @@ void launch_f16_nt_cfg(const GemmArgs& g, hipStream_t s) {
         hipLaunchKernelGGL((k_gemm_f16_nt<BM, BN, BK, WGM, WGN, -1, IGLP>), grid, block, 0, s, g);
 }
 
+// Up to five 128x128 tiles per eight CUs: convh.hip's f16 GEMM, which has smaller tiles and
+// a k split and reads these operands as they lie (no copies).  [8, 4096] x [4096, 4096]
+// 47.1 -> 12.2 us, [512, 1024] x [4096, 1024] (128 tiles) 16.9 -> 12.4, [128, 4096] x [128,
+// 4096] 46.5 -> 11.4, 1536^3 (144) 22.0 -> 19.3; with more tiles the 128x128 kernel re-reads
+// less: [1536, 512] x [1920, 512] (180) 11.7 both, [1536, 512] x [2048, 512] (192) 11.4
+// against 13.7, [1500, 1000] x [2500, 1000] (240) 17.9 against 22.8.
+bool f16_nt_small(int M, int N) {
+    return 8 * (int64_t)((M + 127) / 128) * ((N + 127) / 128) <= 5 * num_cus();
+}
+
 bool launch_f16_nt(const GemmArgs& g, hipStream_t s) {
     const int64_t reach = (int64_t)1 << 31;
     if ((int64_t)(g.M + 256) * g.lda * 2 >= reach || (int64_t)(g.N + 256) * g.ldb * 2 >= reach) return false;
@@ -1355,7 +1365,8 @@ void gemm_impl(const char* name, const Tensor* A, const Tensor* B, const Tensor*
                 const int vec = ((g.lda % 8) == 0 && (g.ldb % 8) == 0 && ((uintptr_t)g.A & 15) == 0 &&
                                  ((uintptr_t)g.B & 15) == 0) ? 1 : 0;
                 int packed = 0;
-                if (!(!transA && transB && vec) && (has_c ? g.c.dt == kF32 && g.c.mode <= 3 : true)) {
+                if ((!(!transA && transB && vec) || f16_nt_small(M, N)) &&
+                    (has_c ? g.c.dt == kF32 && g.c.mode <= 3 : true)) {
                     float* part = nullptr;
                     int nsplit = 0;
                     void* ws = nullptr;

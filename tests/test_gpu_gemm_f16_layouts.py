@@ -33,3 +33,23 @@ def test_gemm_f16_layouts(hip, M, N, K, bias, ta, tb):
             assert_close(y, O.oracle().encode_f32(ref.astype(np.float32), O.F16), O.F16, what="f16")
         else:
             assert_close(y, ref.astype(np.float32), O.F32, what="f32")
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 64, 128), (8, 1000, 4096), (65, 130, 136), (300, 200, 1000), (129, 2100, 512)],
+                         ids=lambda v: str(v))
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+def test_gemm_f16_operands_read_in_place(hip, M, N, K, ta, tb):
+    """K a multiple of eight: an operand with k along its rows is read where it lies, the
+    other from its copy, with one k slice and with several; the bias added once."""
+    rng = np.random.default_rng(M * N + K)
+    a = rng.normal(0, 1, (K, M) if ta else (M, K)).astype(np.float16)
+    b = rng.normal(0, 1 / np.sqrt(K), (N, K) if tb else (K, N)).astype(np.float16)
+    c = rng.normal(0, 1, (N,)).astype(np.float32)
+    ref = (a.T if ta else a).astype(np.float64) @ (b.T if tb else b).astype(np.float64) + c
+    for ydt in ("float16", "float32"):
+        with hip.poisoned():
+            y = hip.gemm(a.view(np.uint16), O.F16, b.view(np.uint16), O.F16, c, O.F32, ydt, 1.0, 1.0, ta, tb)
+        if ydt == "float16":
+            assert_close(y, O.oracle().encode_f32(ref.astype(np.float32), O.F16), O.F16, what="f16")
+        else:
+            assert_close(y, ref.astype(np.float32), O.F32, what="f32")

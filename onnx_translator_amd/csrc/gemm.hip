@@ -787,7 +787,7 @@ struct WoqB {
 // Rows need no alignment beyond a float's (buffer loads take 16 bytes at any 4-byte
 // address).  KT (K % 4 != 0): the elements of a last chunk past K are zeroed before they
 // are stored (in every instance that test took [512, 1024] x [4096, 1024] from 45.7 to
-// 52 us).  [512, 1024] x [1024, 4096] (KN) 124 -> 49.2 us, [300, 1003] x [1001, 1003] 329 ->
+// 52 us).  [512, 1024] x [1024, 4096] (KN) 124 -> 47.3 us, [300, 1003] x [1001, 1003] 329 ->
 // 22.1, [66, 3616] x [3616, 110] 674 -> 19.0 us against the 128x128 kernel without a k
 // split that took them before.
 template <int BM, int BN, int BK, int WGM, int WGN, int YDT, int BQ, int IGLP = -1, bool SPLIT = false, bool KN = false,
@@ -802,6 +802,9 @@ __global__ __launch_bounds__(64 * WGM * WGN) void k_gemm_f32_nt(GemmArgs g, WoqB
     constexpr int EB = BQ ? 1 : 4;                // bytes per B element
     static_assert(CA * NT == BM * CPR && CB * NT == BN * CPR && CA >= 1 && CB >= 1, "tile / thread mismatch");
     static_assert(TM >= 1 && TN >= 1 && BK % 8 == 0, "wave tile");
+    // PARTS: sums of 512 k each, added up at the end (a chain of f32 sums as short as a k
+    // split's: 4.0e-7 from 64 bits at K = 1024 against 5.7e-7 in one chain)
+    constexpr bool PARTS = KN && !SPLIT && BK == 32;
     constexpr int LDN = BN + 4, CPN = BN / 4;     // KN: row pitch and 4-element chunks per row of k
     static_assert(!KN || !BQ, "codes are stored [N, K]");
     __shared__ __attribute__((aligned(16))) float lds[2][KN ? BM * LDK + BK * LDN : (BM + BN) * LDK];
@@ -900,6 +903,13 @@ __global__ __launch_bounds__(64 * WGM * WGN) void k_gemm_f32_nt(GemmArgs g, WoqB
             for (int r = 0; r < 16; r++) acc[i][j][r] = 0.0f;
 
     const int lr = lane & 31, lh = (lane >> 5) * (BK / 2);
+    floatx16 done[PARTS ? TM : 1][PARTS ? TN : 1];
+    if constexpr (PARTS) {
+#pragma unroll
+        for (int i = 0; i < TM; i++)
+#pragma unroll
+            for (int j = 0; j < TN; j++) done[i][j] = acc[i][j];
+    }
     auto compute = [&](int buf) {
         const float* As = &lds[buf][(wm * WTM + lr) * LDK + lh];
         const float* Bs = KN ? &lds[buf][BM * LDK + lh * LDN + wn * WTN + lr] : &lds[buf][(BM + wn * WTN + lr) * LDK + lh];
@@ -944,9 +954,30 @@ __global__ __launch_bounds__(64 * WGM * WGN) void k_gemm_f32_nt(GemmArgs g, WoqB
         compute(cur);
         if constexpr (IGLP >= 0) __builtin_amdgcn_iglp_opt(IGLP);
         store_tile(cur ^ 1, k1);
+        if constexpr (PARTS) {
+            if ((kt + 1) % (512 / BK) == 0) {
+#pragma unroll
+                for (int i = 0; i < TM; i++)
+#pragma unroll
+                    for (int j = 0; j < TN; j++)
+#pragma unroll
+                        for (int r = 0; r < 16; r++) {
+                            done[i][j][r] += acc[i][j][r];
+                            acc[i][j][r] = 0.0f;
+                        }
+            }
+        }
         __syncthreads();
     }
     compute(kt & 1);
+    if constexpr (PARTS) {
+#pragma unroll
+        for (int i = 0; i < TM; i++)
+#pragma unroll
+            for (int j = 0; j < TN; j++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) acc[i][j][r] += done[i][j][r];
+    }
     gfloat* part = (gfloat*)g.Y + (SPLIT ? (int64_t)blockIdx.y * g.M * g.N : 0);
 #pragma unroll
     for (int i = 0; i < TM; i++)
@@ -1239,6 +1270,20 @@ void launch_rows_kernel(const GemmArgs& g, const WoqB& q, int ydt, hipStream_t s
     else hipLaunchKernelGGL((k_gemm_rows<MT, -1, BQ>), grid, block, lds, s, g, q);
 }
 
+// B [K, N] with at least one 128x64 tile per CU: one pass by 8 waves of 32x32 (two per SIMD,
+// k-tiles of 32) in place of two k slices and their reduction, where the tiles' rounds over
+// the CUs are at least 7/8 full: [512, 1024] x [1024, 4096] (256 tiles) 52.5 -> 47.3 us,
+// [1024, 512] x [512, 2048] 38.1 -> 26.5, 2048^3 (512) 155 -> 145; but [640, 2000] x [2000,
+// 4096] (320) 113 against 140.  Long k hides the reduction ([1024, 4096] x [4096, 2048] 158
+// against 167), short k makes it most of the time ([1280, 300] x [300, 2048] (320) 36.3 ->
+// 30.1; by the slopes in k of both the line is near 500).
+inline bool kn_one_pass(int M, int N, int K) {
+    const int64_t cus = num_cus(), tiles = (int64_t)((M + 127) / 128) * ((N + 63) / 64);
+    if (tiles < cus) return false;
+    const int64_t rounds = (tiles + cus - 1) / cus;
+    return 8 * tiles >= 7 * rounds * cus ? K <= 2048 : K <= 384 && rounds == 2;
+}
+
 // probs (f32 [M, N], or null): with a k split, the reduction also takes the
 // rows' softmax into probs (returns 2); otherwise the caller runs the softmax.
 // KN: B [K, N] (transB = 0).
@@ -1262,6 +1307,12 @@ int launch_f32_nt(const GemmArgs& g, const WoqB& q, hipStream_t s, float* probs 
     if (big) {
         launch_nt_kernel<128, 256, 16, 2, 4, BQ, false, KN>(g, q, 0, 1, ydt, s);
         return 1;
+    }
+    if constexpr (KN) {
+        if (kn_one_pass(g.M, g.N, g.K)) {
+            launch_nt_kernel<128, 64, 32, 4, 2, BQ, false, KN>(g, q, 0, 1, ydt, s);
+            return 1;
+        }
     }
     const int kchunk = ((g.K + split - 1) / std::max(split, 1) + 15) / 16 * 16;
     const int nsplit = split > 1 ? (g.K + kchunk - 1) / kchunk : 1;

@@ -75,3 +75,20 @@ def test_gemm_unaligned_bases(hip, tb):
         L.free_tensor(t)
     bt = b.astype(np.float64).T if tb else b.astype(np.float64)
     assert_close(got, (a.astype(np.float64) @ bt).astype(np.float32), O.F32, what="unaligned")
+
+
+@pytest.mark.parametrize("M,N,K", [(2048, 1024, 512), (2047, 1023, 1537), (1025, 2047, 33), (2000, 1100, 383), (1024, 2048, 1030)],
+                         ids=lambda v: str(v))
+def test_gemm_kn_one_pass(hip, M, N, K):
+    """B [K, N] with a 128x64 tile for each CU: one pass in parts of 512 k (one part, a part
+    ending with K, a last part of a few elements).  Three f32 roundings of parts on sums of at
+    most 1537 terms: assert_close's 1e-5."""
+    rng = np.random.default_rng(M + N + K)
+    a = rng.normal(0, 1, (M, K)).astype(np.float32)
+    b = rng.normal(0, 1 / np.sqrt(K), (K, N)).astype(np.float32)
+    c = rng.normal(0, 1, (N,)).astype(np.float32)
+    with hip.poisoned():
+        y = hip.gemm(a, O.F32, b, O.F32, c, O.F32, O.F32, 0.75, 1.5, 0, 0)
+    rows = np.unique(np.r_[rng.choice(M, 60, replace=False), 0, 127, 128, M - 1])
+    ref = 0.75 * (a[rows].astype(np.float64) @ b.astype(np.float64)) + 1.5 * c.astype(np.float64)
+    assert_close(y[rows], ref.astype(np.float32), O.F32, what=f"{M}x{N}x{K}")

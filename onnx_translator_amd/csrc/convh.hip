@@ -412,7 +412,8 @@ void launch_tiles_h(const TilesH& t, const uint4* xp, const uint4* wp, const Epi
 bool launch_conv_f16(const void* x, const void* w, const void* b, int dtb, void* y, int dty, const ConvGeom& cg,
                      hipStream_t s) {
     if ((dty != kF16 && dty != kF32) || (b && dtb != kF32 && dtb != kF16)) return false;
-    if (cg.N < 1 || cg.Cg < 1 || cg.KH < 1 || cg.KW < 1 || cg.group > 65535) return false;
+    // (an image without pixels, whose outputs are all padding, has no copy to index: H * W is divided by)
+    if (cg.N < 1 || cg.Cg < 1 || cg.H < 1 || cg.W < 1 || cg.KH < 1 || cg.KW < 1 || cg.group > 65535) return false;
     // the layout copies live in a workspace, which a captured call may not take
     if (stream_capturing(s)) return false;
     ConvH g;

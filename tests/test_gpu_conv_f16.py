@@ -63,3 +63,16 @@ def test_conv_f16_nonfinite(hip, oracle_lib):
     assert_close(y[:, keep], ref[:, keep], O.F16, what="nonfinite")
     # channel 4 sums to beyond f16: the same infinities
     assert np.array_equal(np.isinf(y[:, 4]), np.isinf(ref[:, 4]))
+
+
+@pytest.mark.parametrize("h,w", [(0, 8), (7, 0)])
+@pytest.mark.parametrize("group", [1, 16], ids=["c16", "depthwise"])
+def test_conv_f16_of_no_pixels(hip, oracle_lib, h, w, group):
+    """No rows or columns, outputs from padding alone: the bias."""
+    rng = np.random.default_rng(h)
+    x = np.zeros((1, 16, h, w), np.float16)
+    wt = rng.normal(0, 1, (16, 16 // group, 3, 3)).astype(np.float16)
+    b = rng.normal(0, 1, 16).astype(np.float32)
+    with hip.poisoned():
+        y = hip.conv(x, O.F16, wt, O.F16, b, O.F32, O.F16, [2, 2, 2, 2], [1, 1], [1, 1], group)
+    assert y.size and np.array_equal(y.view(np.float16), np.broadcast_to(b.astype(np.float16)[:, None, None], y.shape))

@@ -502,11 +502,12 @@ bool launch_split(const void* x, int dtx, void* y, int dty, int64_t L, int G, di
 // one value or none ([64, 21, 4096]: 97 us, 12.3 us so).
 template <int IPT, int CX, int CY, int DIN, int DOUT>
 __global__ __launch_bounds__(CX * CY) void k_softmax_cols(const void* __restrict__ X, int dtx, void* __restrict__ Y,
-                                                               int dty, int64_t L, int64_t inner, uint32_t nbx) {
+                                                               int dty, int64_t L, int64_t inner, int64_t r0,
+                                                               uint32_t nbx) {
     __shared__ double red[CY][CX];
     const int cx = threadIdx.x & (CX - 1), ry = threadIdx.x / CX;
     const int64_t bo = blockIdx.x / nbx;
-    const int64_t r = (int64_t)(blockIdx.x - bo * nbx) * CX + cx;
+    const int64_t r = r0 + (int64_t)(blockIdx.x - bo * nbx) * CX + cx;
     const bool live = r < inner;
     const int64_t base = bo * L * inner + (live ? r : 0);
     double v[IPT > 0 ? IPT : 1];
@@ -567,17 +568,21 @@ template <int DIN, int DOUT>
 void launch_cols(const void* x, int dtx, void* y, int dty, int64_t outer, int64_t L, int64_t inner, hipStream_t s) {
     const bool few = L <= 64;
     const int cx = few ? 64 : 32, cy = few ? 4 : 32;
-    const uint32_t nbx = (uint32_t)((inner + cx - 1) / cx);
     const int64_t ipt = (L + cy - 1) / cy;
     const dim3 b(cx * cy);
-    // one grid dimension holds every (outer, column block): slices of at most 2^30 blocks
-    const int64_t per = std::max<int64_t>(1, ((int64_t)1 << 30) / nbx);
-    for (int64_t o = 0; o < outer; o += per) {
+    // One grid dimension holds every (outer, column block).  The runtime takes fewer than 2^32
+    // work-items in it: slices of at most 2^31, of whole outers or of one outer's columns.
+    const int64_t most = ((int64_t)1 << 31) / (cx * cy), all = (inner + cx - 1) / cx, nb = std::min(all, most);
+    const int64_t per = std::max<int64_t>(1, most / all);
+    for (int64_t o = 0; o < outer; o += per)
+    for (int64_t cb = 0; cb < all; cb += nb) {
+        const uint32_t nbx = (uint32_t)std::min(nb, all - cb);
+        const int64_t r0 = cb * cx;
         const dim3 g((unsigned)(std::min(per, outer - o) * nbx));
         const char* xo = (const char*)x + (size_t)(o * L * inner) * dt_bytes(dtx);
         char* yo = (char*)y + (size_t)(o * L * inner) * dt_bytes(dty);
 #define SM_COLS(I, CX, CY) \
-    hipLaunchKernelGGL((k_softmax_cols<I, CX, CY, DIN, DOUT>), g, b, 0, s, xo, dtx, yo, dty, L, inner, nbx)
+    hipLaunchKernelGGL((k_softmax_cols<I, CX, CY, DIN, DOUT>), g, b, 0, s, xo, dtx, yo, dty, L, inner, r0, nbx)
         if (few) {
             if (ipt <= 2) SM_COLS(2, 64, 4);
             else if (ipt <= 4) SM_COLS(4, 64, 4);

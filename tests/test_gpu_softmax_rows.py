@@ -78,3 +78,39 @@ def test_gemm_softmax_same_rows(hip, M, N):
         assert_bitexact(hip.dev_read(p2, O.F32), hip.dev_read(p1, O.F32), O.F32, what="probabilities")
     finally:
         dev.free()
+
+
+@pytest.mark.parametrize("shape,dtype", [((1 << 24, 2, 2), "float32"), (((1 << 22) + 3, 65, 1, 2), "float16"),
+                                         ((1, 2, (1 << 30) + 5), "float16")], ids=["outer24", "outer22", "inner30"])
+def test_softmax_columns_in_slices(hip, shape, dtype):
+    """More column blocks than one launch holds, by the outer or the inner dimension: every
+    value against torch's float32 softmax (1e-6 for f32 outputs of at most 1; one unit in the
+    last place of f16, 2^-11 of values of at most 1)."""
+    import torch
+    from tests.test_gpu_qconv import _bind
+    L = hip.lib
+    _bind(L)
+    L.softmax_forward.argtypes = [O.PT, O.PT, ctypes.c_int]
+    g = torch.Generator(device="cuda")
+    g.manual_seed(3)
+    x = torch.empty(shape, dtype=getattr(torch, dtype), device="cuda").normal_(0, 2, generator=g)
+    y = torch.full_like(x, float("nan"))
+    ts = [L.tensor_wrap_device(ctypes.c_void_p(t.data_ptr()), (ctypes.c_int * len(shape))(*shape), len(shape),
+                               O.F32 if dtype == "float32" else O.F16) for t in (x, y)]
+    torch.cuda.synchronize()
+    L.tensor_ops_hip_clear_error()
+    L.softmax_forward(*ts, 1)
+    assert not hip.last_error(), hip.last_error()
+    hip.lib.tensor_ops_hip_sync()
+    for t in ts:
+        L.free_tensor(t)
+    # in pieces along the longest dimension
+    dim = int(np.argmax(shape))
+    step = 1 << 22 if shape[1] > 2 else 1 << 24
+    for a in range(0, shape[dim], step):
+        n = min(step, shape[dim] - a)
+        want = torch.softmax(x.narrow(dim, a, n).float(), 1)
+        d = (y.narrow(dim, a, n).float() - want).abs().max().item()
+        assert d <= (1e-6 if dtype == "float32" else 2.0 ** -11), (a, d)
+    del x, y
+    torch.cuda.empty_cache()

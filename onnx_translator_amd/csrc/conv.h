@@ -50,10 +50,9 @@ bool launch_conv_depthwise(const void* x, int dtx, const void* w, const void* b,
 // The layers launch_conv_depthwise takes, by their shape alone.
 bool conv_depthwise_shape(const ConvGeom& g);
 
-
 // float16 X and W on the f16 matrix cores (convh.hip): f16 / f32 output, f32 / f16 or
-// no bias, any groups.  False when the layer is outside the plan (nothing launched;
-// with the error set when the workspace could not be had).
+// no bias, any groups.  False, with nothing launched and no error, when the layer is outside
+// the plan or there is no memory for the copies.
 bool launch_conv_f16(const void* x, const void* w, const void* b, int dtb, void* y, int dty, const ConvGeom& g,
                      hipStream_t s);
 

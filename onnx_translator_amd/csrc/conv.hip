@@ -1165,6 +1165,7 @@ __global__ __launch_bounds__(256) void k_conv_splitk_reduce4(const float* __rest
     *(float4*)(Y + i) = make_float4(v[0], v[1], v[2], v[3]);
 }
 
+// False, with nothing launched and no error, without memory for the slices.
 template <int BM, int BP, int BK, int WGM, int WGN, int MODE, int XQ = 0, int DEPTH = 1>
 bool launch_conv_split_cfg(const float* x, const float* w, const float* b, float* y, const ConvTiled& g, int group,
                            uint32_t xbytes, uint32_t wbytes, int nsplit_req, ConvEpi epi, ConvXQ xq, hipStream_t s) {
@@ -1172,7 +1173,7 @@ bool launch_conv_split_cfg(const float* x, const float* w, const float* b, float
     const int kchunk = ((g.Kg + nsplit_req - 1) / nsplit_req + BK - 1) / BK * BK;
     const int nsplit = (g.Kg + kchunk - 1) / kchunk;
     const int64_t total = (int64_t)g.P * g.M;
-    float* part = (float*)pool_alloc((size_t)nsplit * total * sizeof(float));
+    float* part = (float*)pool_alloc((size_t)nsplit * total * sizeof(float), true);
     if (!part) return false;
     const dim3 grid((g.P + BP - 1) / BP, (g.Mg + BM - 1) / BM, group * nsplit), block(64 * WGM * WGN);
     hipLaunchKernelGGL((k_conv_tiled<BM, BP, BK, WGM, WGN, MODE, kF32, true, XQ, DEPTH>), grid, block, 0, s, x, w, b, part,
@@ -1305,25 +1306,24 @@ bool launch_conv_tiled_xq(const void* x, const void* w, const void* b, int dtb, 
         // (an XQ launch always has an f32 output and an f32 or no bias)
         const float* bf = (const float*)b;
         float* yf = (float*)y;
+        bool done;
         if (direct)
-            return launch_conv_split_cfg<64, 256, 16, 2, 4, 1, XQ>(xf, wf, bf, yf, g, cg.group, ux, uw, split, epi, xq, s);
-        if (plan == kT64x64)
-            return launch_conv_split_cfg<64, 64, 16, 2, 2, 2, XQ, 2>(xf, wf, bf, yf, g, cg.group, ux, uw, split, epi, xq,
-                                                                     s);
-        if (plan == kT64x128)
-            return launch_conv_split_cfg<64, 128, 16, 2, 4, 2, XQ, 2>(xf, wf, bf, yf, g, cg.group, ux, uw, split, epi, xq,
-                                                                      s);
-        if (plan == kT128x128)
-            return launch_conv_split_cfg<128, 128, 16, 4, 4, 2, XQ, 2>(xf, wf, bf, yf, g, cg.group, ux, uw, split, epi,
-                                                                       xq, s);
-        if (plan == kT128x256)
-            return launch_conv_split_cfg<128, 256, 16, 2, 8, 2, XQ, 2>(xf, wf, bf, yf, g, cg.group, ux, uw, split, epi,
-                                                                       xq, s);
-        if (plan == kT64x256)
-            return launch_conv_split_cfg<64, 256, 16, 2, 4, 2, XQ>(xf, wf, bf, yf, g, cg.group, ux, uw, split, epi, xq, s);
-        if (g.Kg <= 256)
-            return launch_conv_split_cfg<64, 256, 8, 2, 4, 0, XQ>(xf, wf, bf, yf, g, cg.group, ux, uw, split, epi, xq, s);
-        return launch_conv_split_cfg<64, 256, 16, 2, 8, 0, XQ>(xf, wf, bf, yf, g, cg.group, ux, uw, split, epi, xq, s);
+            done = launch_conv_split_cfg<64, 256, 16, 2, 4, 1, XQ>(xf, wf, bf, yf, g, cg.group, ux, uw, split, epi, xq, s);
+        else if (plan == kT64x64)
+            done = launch_conv_split_cfg<64, 64, 16, 2, 2, 2, XQ, 2>(xf, wf, bf, yf, g, cg.group, ux, uw, split, epi, xq, s);
+        else if (plan == kT64x128)
+            done = launch_conv_split_cfg<64, 128, 16, 2, 4, 2, XQ, 2>(xf, wf, bf, yf, g, cg.group, ux, uw, split, epi, xq, s);
+        else if (plan == kT128x128)
+            done = launch_conv_split_cfg<128, 128, 16, 4, 4, 2, XQ, 2>(xf, wf, bf, yf, g, cg.group, ux, uw, split, epi, xq, s);
+        else if (plan == kT128x256)
+            done = launch_conv_split_cfg<128, 256, 16, 2, 8, 2, XQ, 2>(xf, wf, bf, yf, g, cg.group, ux, uw, split, epi, xq, s);
+        else if (plan == kT64x256)
+            done = launch_conv_split_cfg<64, 256, 16, 2, 4, 2, XQ>(xf, wf, bf, yf, g, cg.group, ux, uw, split, epi, xq, s);
+        else if (g.Kg <= 256)
+            done = launch_conv_split_cfg<64, 256, 8, 2, 4, 0, XQ>(xf, wf, bf, yf, g, cg.group, ux, uw, split, epi, xq, s);
+        else
+            done = launch_conv_split_cfg<64, 256, 16, 2, 8, 0, XQ>(xf, wf, bf, yf, g, cg.group, ux, uw, split, epi, xq, s);
+        if (done) return true;      // else the same tiles without slices
     }
     if (direct && g.Kg <= 64)
         // shallow 1x1 layers: BK 8 (the config-4 1x1, K = 64: 42.8 -> 42.1 us over six A/B

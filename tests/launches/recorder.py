@@ -43,6 +43,8 @@ class Recorder:
         L.tensor_wrap_device.restype = PT
         L.tensor_wrap_device.argtypes = [ctypes.c_void_p, ctypes.POINTER(ci), ci, ci]
         L.free_tensor.argtypes = [PT]
+        L.create_tensor_device_empty.restype = PT
+        L.create_tensor_device_empty.argtypes = [ctypes.POINTER(ci), ci, ci]
         L.tensor_ops_hip_last_error.restype = ctypes.c_char_p
         L.conv2d_forward.argtypes = [PT] * 4 + [ctypes.POINTER(O.CConvParams)]
         L.conv2d_fused_forward.argtypes = [PT] * 4 + [ci, PT, ctypes.POINTER(O.CConvParams)]
@@ -59,6 +61,12 @@ class Recorder:
         t = self.lib.tensor_wrap_device(self._at + offset, (ctypes.c_int * len(shape))(*shape), len(shape), dt)
         self._at += 1 << 36
         return t
+
+    def no_memory(self, on):
+        """Device allocations fail from here on (and the pool's cached buffers are given up)."""
+        self.lib.stub_malloc_limit(0 if on else (1 << 64) - 1)
+        if on:      # an allocation that fails
+            assert not self.lib.create_tensor_device_empty(O._ints([1 << 30]), 1, O.F32)
 
     def call(self, fn, *args):
         """(launches, error) of one call of the library's fn."""

@@ -42,3 +42,39 @@ def test_softmax_columns_in_slices(rec, shape, threads):
     cols = 64 if threads == 256 else 32
     assert all(l.block == threads for l in launches)
     assert sum(l.grid[0] for l in launches) == shape[0] * -(-shape[2] // cols)
+
+
+# f32: direct 1x1, 64x64, 128x256, 64x256 and per-pixel plans, all with slices of k
+SPLIT_CONVS = [((1, 1024, 14, 14), 256, (1, 1), 1), ((1, 512, 7, 7), 512, (3, 3), 1), ((8, 256, 28, 28), 128, (3, 3), 2),
+               ((2, 250, 30, 30), 64, (3, 3), 1), ((1, 19, 14, 14), 30, (3, 3), 1), ((64, 512, 7, 7), 512, (3, 3), 1)]
+
+
+@pytest.mark.parametrize("codes", [None, O.U8], ids=["f32", "codes"])
+@pytest.mark.parametrize("xs,m,k,s", SPLIT_CONVS, ids=["x".join(map(str, c[0])) for c in SPLIT_CONVS])
+def test_conv_split_without_memory(rec, xs, m, k, s, codes):
+    """No memory for the slices: the same tiles in one pass, and no error."""
+    args = (xs, m, k, (k[0] // 2,) * 4, (s, s))
+    with_memory = rec.conv(*args, codes=codes)
+    rec.no_memory(True)
+    try:
+        without = rec.conv(*args, codes=codes)
+    finally:
+        rec.no_memory(False)
+    split = kernels(with_memory)
+    assert kernels(without) == ["k_conv_tiled"]
+    if split != ["k_conv_tiled"]:
+        assert split[0] == "k_conv_tiled" and split[1].startswith("k_conv_splitk_reduce")
+    else:
+        assert xs[1] == 19        # K below two slices
+
+
+def test_workspace_paths_without_memory(rec):
+    """f16 convolution and Gemm copies, f32 Gemm slices: the path that needs none."""
+    rec.no_memory(True)
+    try:
+        assert kernels(rec.conv((32, 128, 28, 28), 128, (3, 3), (1, 1, 1, 1), dt=O.F16)) == ["k_conv_mfma_f32"]
+        assert kernels(rec.gemm(512, 1000, 1024, tb=0, dt=O.F16)) == ["k_gemm_mfma_f16"]
+        assert kernels(rec.gemm(8, 4096, 4096, dt=O.F16)) == ["k_gemm_f16_nt"]
+        assert kernels(rec.gemm(128, 1000, 1024)) == ["k_gemm_f32_nt"]
+    finally:
+        rec.no_memory(False)

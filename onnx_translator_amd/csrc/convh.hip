@@ -477,7 +477,7 @@ bool launch_conv_f16(const void* x, const void* w, const void* b, int dtb, void*
 constexpr int kGemmHMinK = 128;
 
 int launch_gemm_f16_packed(const GemmH& q, hipStream_t s, float** part, int* nsplit, void** ws) {
-    if ((q.dty != kF16 && q.dty != kF32) || q.M < 1 || q.N < 1 || q.K < kGemmHMinK || stream_capturing(s)) return 0;
+    if ((q.dty != kF16 && q.dty != kF32) || q.M < 1 || q.N < 1 || q.K < kGemmHMinK) return 0;
     const int64_t KC = ((int64_t)q.K + 7) / 8, reach = (int64_t)1 << 31;
     const int64_t ab = (int64_t)q.M * KC * 16, bb = (int64_t)q.N * KC * 16, total = (int64_t)q.M * q.N;
     if (ab >= reach || bb >= reach || total >= reach / 4) return 0;
@@ -488,7 +488,7 @@ int launch_gemm_f16_packed(const GemmH& q, hipStream_t s, float** part, int* nsp
     const bool a_own = !q.ta && q.K % 8 == 0 && ((uintptr_t)q.A & 15) == 0;
     const bool b_own = q.tb && q.K % 8 == 0 && ((uintptr_t)q.B & 15) == 0;
     const int64_t ac = a_own ? 0 : up(ab), bc = b_own ? 0 : up(bb);
-    char* w = nullptr;
+    char* w = nullptr;      // (none to be had under graph capture: only calls without copies and slices then)
     if (ac + bc + pb && !(w = (char*)pool_alloc((size_t)(ac + bc + pb), true))) return 0;
     const uint4 *ap = a_own ? (const uint4*)q.A : (const uint4*)w, *bp = b_own ? (const uint4*)q.B : (const uint4*)(w + ac);
     ConvH g;

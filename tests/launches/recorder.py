@@ -68,6 +68,10 @@ class Recorder:
         if on:      # an allocation that fails
             assert not self.lib.create_tensor_device_empty(O._ints([1 << 30]), 1, O.F32)
 
+    def capturing(self, on):
+        """The stream counts as being captured into a graph."""
+        self.lib.stub_capturing(1 if on else 0)
+
     def call(self, fn, *args):
         """(launches, error) of one call of the library's fn."""
         self._take()

@@ -384,3 +384,89 @@ def test_capture_first_on_fresh_stream(hip, oracle_lib):
         for p in keep:
             L.free_tensor(p)
         L.tensor_ops_hip_set_stream(None)
+
+
+def test_workspace_calls_under_capture(hip, oracle_lib):
+    """Calls that eagerly take a workspace (f16 convolution copies, f16 Gemm copies and k
+    slices, f32 Gemm slices), captured: the path without one, against the oracle (assert_close:
+    one unit in the last place of f16, 1e-5 for f32).  An f16 Gemm that needs none runs the
+    eager kernel: its bits.  Inputs change between replays, with eager calls in between."""
+    import torch
+    torch.cuda.init()
+    side = torch.cuda.Stream()
+    L = hip.lib
+    L.gemm_forward.argtypes = [O.PT] * 4 + [ctypes.c_float, ctypes.c_float, ctypes.c_int, ctypes.c_int]
+    L.conv2d_forward.argtypes = [O.PT] * 4 + [ctypes.POINTER(O.CConvParams)]
+    L.tensor_ops_hip_set_stream(ctypes.c_void_p(side.cuda_stream))
+    keep = []
+    wrap = _wrapper(L, keep)
+    rng = np.random.default_rng(71)
+    ints = [O._ints([1, 1, 1, 1]), O._ints([1, 1]), O._ints([1, 1])]
+    prm = O.CConvParams()
+    prm.pads, prm.strides, prm.dilations = [ctypes.cast(v, ctypes.POINTER(ctypes.c_int)) for v in ints]
+    prm.group = 1
+    # name: input shapes (f16 but for f32 biases and "f32"), output shape, transB
+    gemms = {"nn": ((70, 300), (300, 130), (70, 130), 0), "slices": ((8, 2048), (500, 2048), (8, 500), 1),
+             "in_place": ((300, 200), (64, 200), (300, 64), 1), "f32": ((70, 1024), (1000, 1024), (70, 1000), 1)}
+    xs, ws = (2, 24, 13, 11), (20, 24, 3, 3)
+
+    def draw(shape, dt):
+        return rng.normal(0, 0.3, shape).astype(dt)
+
+    try:
+        with torch.cuda.stream(side):
+            dev, t, out = {}, {}, {}
+            for n, (a, b, y, _) in gemms.items():
+                ht, dt = (torch.float32, O.F32) if n == "f32" else (torch.float16, O.F16)
+                dev[n] = [torch.empty(a, dtype=ht, device="cuda"), torch.empty(b, dtype=ht, device="cuda"),
+                          torch.empty(y[1], dtype=torch.float32, device="cuda")]
+                out[n] = torch.empty(y, dtype=ht, device="cuda")
+                t[n] = [wrap(v, list(v.shape), d) for v, d in zip(dev[n] + [out[n]], (dt, dt, O.F32, dt))]
+            dev["conv"] = [torch.empty(xs, dtype=torch.float16, device="cuda"), torch.empty(ws, dtype=torch.float16, device="cuda"),
+                           torch.empty(ws[0], dtype=torch.float32, device="cuda")]
+            out["conv"] = torch.empty((2, 20, 13, 11), dtype=torch.float16, device="cuda")
+            t["conv"] = [wrap(v, list(v.shape), d) for v, d in zip(dev["conv"] + [out["conv"]], (O.F16, O.F16, O.F32, O.F16))]
+
+            def calls():
+                for n, g in gemms.items():
+                    L.gemm_forward(*t[n], 1.0, 1.0, 0, g[3])
+                L.conv2d_forward(*t["conv"], ctypes.byref(prm))
+
+            L.tensor_ops_hip_clear_error()
+            graph = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(graph, stream=side):
+                calls()
+            assert not hip.last_error(), hip.last_error()
+            for r in range(3):
+                host = {n: [draw(tuple(v.shape), np.float32 if v.dtype == torch.float32 else np.float16) for v in vs]
+                        for n, vs in dev.items()}
+                for n, vs in dev.items():
+                    for v, h in zip(vs, host[n]):
+                        v.copy_(torch.from_numpy(h))
+                for v in out.values():
+                    v.fill_(float("nan"))
+                torch.cuda.synchronize()
+                graph.replay()
+                torch.cuda.synchronize()
+                got = {n: v.cpu().numpy() for n, v in out.items()}
+                calls()
+                torch.cuda.synchronize()
+                assert not hip.last_error(), hip.last_error()
+                print(f"workspace calls: replay {r}", flush=True)
+                for n, v in out.items():
+                    eager = v.cpu().numpy()
+                    a, b, c = host[n]
+                    dt = O.F32 if n == "f32" else O.F16
+                    if n == "conv":
+                        ref = oracle_lib.conv(a, O.F16, b, O.F16, c, O.F32, O.F16, [1, 1, 1, 1], [1, 1], [1, 1], 1)
+                    else:
+                        ref = oracle_lib.gemm(a, dt, b, dt, c, O.F32, dt, 1.0, 1.0, 0, gemms[n][3])
+                    view = (lambda z: z) if dt == O.F32 else (lambda z: z.view(np.uint16))
+                    assert_close(view(got[n]), ref, dt, what=f"replay {r} {n}")
+                    assert_close(view(eager), ref, dt, what=f"eager {r} {n}")
+                    if n == "in_place":
+                        assert_bitexact(view(got[n]), view(eager), O.F16, what=f"replay {r} {n}")
+    finally:
+        for p in keep:
+            L.free_tensor(p)
+        L.tensor_ops_hip_set_stream(None)

@@ -78,3 +78,17 @@ def test_workspace_paths_without_memory(rec):
         assert kernels(rec.gemm(128, 1000, 1024)) == ["k_gemm_f32_nt"]
     finally:
         rec.no_memory(False)
+
+
+@pytest.mark.parametrize("m,n,k", [(1000, 1000, 128), (300, 64, 200), (1, 64, 136)])
+def test_gemm_f16_in_place_under_capture(rec, m, n, k):
+    """Operands read where they lie and one k slice need no workspace: the captured call runs
+    the eager call's kernel.  Copies need one: the kernel without them."""
+    eager, copies = rec.gemm(m, n, k, dt=O.F16), rec.gemm(m, n, k, tb=0, dt=O.F16)
+    rec.capturing(True)
+    try:
+        assert rec.gemm(m, n, k, dt=O.F16) == eager and kernels(eager) == ["k_convh"]
+        assert kernels(copies)[-1] == "k_convh" and kernels(rec.gemm(m, n, k, tb=0, dt=O.F16)) == ["k_gemm_mfma_f16"]
+        assert kernels(rec.conv((8, 64, 28, 28), 64, (3, 3), (1, 1, 1, 1), dt=O.F16)) == ["k_conv_mfma_f32"]
+    finally:
+        rec.capturing(False)

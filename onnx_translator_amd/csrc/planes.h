@@ -108,7 +108,8 @@ inline int row_threads_log2(int n) {
 }
 
 // Fills in the tiles for strips of R output rows (extra: floats of LDS per plane besides
-// its rows).  H, W, ..., dw, C, M and planes are set; false when a row is too wide.
+// its rows).  H, W, ..., dw, C, M and planes are set; false when a row is too wide or the
+// blocks are more than one launch holds.
 inline bool plan_planes(PlaneTiles& p, int R, int extra) {
     const int64_t pw = (int64_t)(p.OW - 1) * p.sw + (int64_t)(p.KW - 1) * p.dw + 1;
     auto rows = [&](int64_t tr) { return (tr - 1) * p.sh + (int64_t)(p.KH - 1) * p.dh + 1; };
@@ -128,6 +129,8 @@ inline bool plan_planes(PlaneTiles& p, int R, int extra) {
         const int64_t fit = kPlaneTile / ((int64_t)p.PR * p.PW + extra);
         p.np = (int)std::max<int64_t>(1, std::min<int64_t>(fit, p.planes / (2 * num_cus())));
     }
+    // the runtime takes fewer than 2^32 work-items per grid dimension
+    if ((p.planes + (int64_t)p.np - 1) / p.np * p.tiles * kPlaneThreads >= (int64_t)1 << 32) return false;
     p.lxl = row_threads_log2(p.PW);
     p.lxo = row_threads_log2(p.OW);
     p.cc = (p.PW + (1 << p.lxl) - 1) >> p.lxl;

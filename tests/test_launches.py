@@ -92,3 +92,15 @@ def test_gemm_f16_in_place_under_capture(rec, m, n, k):
         assert kernels(rec.conv((8, 64, 28, 28), 64, (3, 3), (1, 1, 1, 1), dt=O.F16)) == ["k_conv_mfma_f32"]
     finally:
         rec.capturing(False)
+
+
+@pytest.mark.parametrize("k,pads,dil", [((31, 31), 15, 1), ((2, 2), 25, 50)], ids=["31x31", "dilated"])
+@pytest.mark.parametrize("dt", [O.F32, O.F16, O.U8], ids=["f32", "f16", "codes"])
+def test_depthwise_launch_within_the_work_items(rec, k, pads, dil, dt):
+    """Many planes of one pixel under a wide window, few to a block: the depthwise kernel's
+    blocks would be past 2^32 work-items; the layer runs all the same."""
+    pads = (pads,) * 4
+    r = rec.conv((1 << 28, 1, 1, 1), 1, k, pads, (1, 1), (dil, dil), 1, dt=dt, codes=O.U8 if dt == O.U8 else None)
+    assert len(kernels(r)) == 1
+    few = rec.conv((1 << 10, 1, 1, 1), 1, k, pads, (1, 1), (dil, dil), 1, dt=dt, codes=O.U8 if dt == O.U8 else None)
+    assert kernels(few) == ["k_conv_dw"]

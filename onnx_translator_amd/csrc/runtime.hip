@@ -727,11 +727,21 @@ static bool sync_copy_under_capture(const char* name) {
 // order), the stream is waited for and the bytes are copied on.  The runtime's copy to
 // pageable memory goes through its staging and a copy engine instead: 4 KB 24 -> 14.6 us,
 // and 88 us less per forward of the one-image residual network with its two outputs.
-// False: not taken (nothing enqueued).
+// Memory that is not the library's own may lie on another device, which a kernel here
+// cannot be sure to reach: the runtime's copy takes it.  False: not taken (nothing enqueued).
 constexpr size_t kSmallResult = 256 << 10;
 
-static bool small_result(const Tensor* t, void* host_dst, size_t b, bool& ok) {
-    if (b > kSmallResult || !g_result_copy) return false;
+static bool on_library_device(const void* p, Mem m) {
+    if (m == Mem::kDevOwned) return true;
+    hipPointerAttribute_t a;
+    memset(&a, 0, sizeof a);
+    if (hipPointerGetAttributes(&a, p) == hipSuccess) return a.type == hipMemoryTypeDevice && a.device == S().dev;
+    (void)hipGetLastError();
+    return false;
+}
+
+static bool small_result(const Tensor* t, Mem m, void* host_dst, size_t b, bool& ok) {
+    if (b > kSmallResult || !g_result_copy || !on_library_device(t->data, m)) return false;
     void* pin = pinned_alloc(b);
     if (!pin) return false;
     ok = g_result_copy(t->data, pin, b, stream()) && check_hip(hipStreamSynchronize(stream()), "stream synchronize");
@@ -744,10 +754,11 @@ int tensor_to_host(const Tensor* t, void* host_dst) {
     if (!tensor_sane(t, "tensor_to_host") || !host_dst) return -1;
     const size_t b = tensor_bytes(t);
     if (!b) return 0;
-    if (is_dev(classify(t->data))) {
+    const Mem m = classify(t->data);
+    if (is_dev(m)) {
         if (sync_copy_under_capture("tensor_to_host")) return -1;
         bool ok = false;
-        if (small_result(t, host_dst, b, ok)) return ok ? 0 : -1;
+        if (small_result(t, m, host_dst, b, ok)) return ok ? 0 : -1;
         if (!check_hip(hipMemcpyAsync(host_dst, t->data, b, hipMemcpyDeviceToHost, stream()), "D2H copy") ||
             !check_hip(hipStreamSynchronize(stream()), "stream synchronize"))
             return -1;

@@ -24,6 +24,7 @@ std::string log_;
 hipError_t last = hipSuccess;
 size_t malloc_limit = ~size_t(0);
 bool capturing = false;
+int pointer_device = -1;                // of memory that the library does not own; -1: not known
 uintptr_t next_address = uintptr_t(1) << 44;
 
 struct Config {
@@ -38,6 +39,7 @@ extern "C" {
 // ---- what the tests set and read
 void stub_malloc_limit(size_t bytes) { malloc_limit = bytes; }
 void stub_capturing(int on) { capturing = on != 0; }
+void stub_pointer_device(int d) { pointer_device = d; }
 // The launches since the last call, one per line: kernel|grid x y z|block.  Freed by the caller.
 char* stub_launches() {
     std::lock_guard<std::mutex> g(mu);
@@ -103,7 +105,12 @@ hipError_t hipHostMalloc(void** p, size_t bytes, unsigned) {
 }
 hipError_t hipHostFree(void* p) { free(p); return hipSuccess; }
 hipError_t hipGetSymbolAddress(void** p, const void*) { return hipMalloc(p, 4096); }
-hipError_t hipPointerGetAttributes(hipPointerAttribute_t*, const void*) { return last = hipErrorInvalidValue; }
+hipError_t hipPointerGetAttributes(hipPointerAttribute_t* a, const void*) {
+    if (pointer_device < 0) return last = hipErrorInvalidValue;
+    a->type = hipMemoryTypeDevice;
+    a->device = pointer_device;
+    return hipSuccess;
+}
 hipError_t hipMemcpy(void*, const void*, size_t, hipMemcpyKind) { return hipSuccess; }
 hipError_t hipMemcpyAsync(void*, const void*, size_t, hipMemcpyKind, hipStream_t) { return hipSuccess; }
 hipError_t hipMemsetAsync(void*, int, size_t, hipStream_t) { return hipSuccess; }

@@ -72,6 +72,16 @@ class Recorder:
         """The stream counts as being captured into a graph."""
         self.lib.stub_capturing(1 if on else 0)
 
+    def to_host(self, shape, dt, owned=False, device=-1):
+        """(launches, error) of reading a tensor of the library's own memory, or of memory that
+        the runtime says lies on a device (-1: that it does not know)."""
+        t = self.lib.create_tensor_device_empty(O._ints(shape), len(shape), dt) if owned else self.tensor(shape, dt)
+        self.lib.stub_pointer_device(device)
+        try:
+            return self.call("tensor_to_host", t, ctypes.create_string_buffer(1 << 16))
+        finally:
+            self.lib.stub_pointer_device(-1)
+
     def call(self, fn, *args):
         """(launches, error) of one call of the library's fn."""
         self._take()

@@ -104,3 +104,11 @@ def test_depthwise_launch_within_the_work_items(rec, k, pads, dil, dt):
     assert len(kernels(r)) == 1
     few = rec.conv((1 << 10, 1, 1, 1), 1, k, pads, (1, 1), (dil, dil), 1, dt=dt, codes=O.U8 if dt == O.U8 else None)
     assert kernels(few) == ["k_conv_dw"]
+
+
+def test_small_result_of_another_device(rec):
+    """Results that a kernel here may not reach go through the runtime's copy."""
+    assert kernels(rec.to_host((1000,), O.F32, owned=True)) == ["k_result"]
+    assert kernels(rec.to_host((1000,), O.F32, device=0)) == ["k_result"]
+    assert kernels(rec.to_host((1000,), O.F32, device=1)) == []
+    assert kernels(rec.to_host((1000,), O.F32, device=-1)) == []

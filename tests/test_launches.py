@@ -112,3 +112,9 @@ def test_small_result_of_another_device(rec):
     assert kernels(rec.to_host((1000,), O.F32, device=0)) == ["k_result"]
     assert kernels(rec.to_host((1000,), O.F32, device=1)) == []
     assert kernels(rec.to_host((1000,), O.F32, device=-1)) == []
+
+
+def test_small_results_only(rec):
+    """The runtime's copy is the slower one up to 16 KB only."""
+    assert kernels(rec.to_host((4096,), O.F32, owned=True)) == ["k_result"]
+    assert kernels(rec.to_host((16385,), O.U8, owned=True)) == []

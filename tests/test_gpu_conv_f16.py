@@ -26,6 +26,13 @@ CASES = [
     ("tiles_64x128", (8, 16, 56, 56), 72, (3, 3), (1, 1, 1, 1), (1, 1), (1, 1), 1),
     ("tiles_128x128", (24, 8, 54, 52), 130, (1, 1), (0, 0, 0, 0), (1, 1), (1, 1), 1),
     ("oh_odd_width2", (2, 16, 10, 5), 8, (3, 3), (1, 1, 1, 1), (1, 1), (1, 1), 1),
+    # many k-tiles through the rings of LDS slots: every remainder of three slots (18, 19 and
+    # 20 tiles of 64x128) and of two (2 and 11 tiles of 128x128)
+    ("ring_64x128_18", (32, 128, 28, 28), 128, (3, 3), (1, 1, 1, 1), (1, 1), (1, 1), 1),
+    ("ring_64x128_19", (8, 48, 56, 56), 72, (5, 5), (2, 2, 2, 2), (1, 1), (1, 1), 1),
+    ("ring_64x128_20", (8, 136, 56, 56), 72, (3, 3), (1, 1, 1, 1), (1, 1), (1, 1), 1),
+    ("ring_128x128_2", (24, 120, 54, 52), 130, (1, 1), (0, 0, 0, 0), (1, 1), (1, 1), 1),
+    ("ring_128x128_11", (24, 72, 54, 52), 130, (3, 3), (1, 1, 1, 1), (1, 1), (1, 1), 1),
 ]
 
 
@@ -63,6 +70,23 @@ def test_conv_f16_nonfinite(hip, oracle_lib):
     assert_close(y[:, keep], ref[:, keep], O.F16, what="nonfinite")
     # channel 4 sums to beyond f16: the same infinities
     assert np.array_equal(np.isinf(y[:, 4]), np.isinf(ref[:, 4]))
+
+
+@pytest.mark.parametrize("odt", [O.F16, O.F32], ids=["f16", "f32"])
+@pytest.mark.parametrize("sub", ["x", "w", "y"])
+def test_conv_f16_subnormals(hip, oracle_lib, sub, odt):
+    """Subnormal halves in X or in W count with their value, and subnormal results are rounded
+    to the subnormals' spacing."""
+    rng = np.random.default_rng(17)
+    tiny = lambda shape: (rng.integers(-1023, 1024, shape) * 2.0 ** -24).astype(np.float16)
+    xs, ws = (2, 24, 9, 8), (10, 24, 3, 3)
+    x = tiny(xs) if sub == "x" else rng.normal(0, 0.02 if sub == "y" else 1, xs).astype(np.float16)
+    w = tiny(ws) if sub == "w" else rng.normal(0, 5e-5 if sub == "y" else 1, ws).astype(np.float16)
+    args = ([1, 1, 1, 1], [1, 1], [1, 1], 1)
+    y = hip.conv(x, O.F16, w, O.F16, None, O.F32, odt, *args)
+    ref = oracle_lib.conv(x, O.F16, w, O.F16, None, O.F32, odt, *args)
+    assert_close(y, ref, odt, what=sub)
+    assert np.count_nonzero(ref) > ref.size // 2
 
 
 @pytest.mark.parametrize("h,w", [(0, 8), (7, 0)])

@@ -1,9 +1,9 @@
 """gemm_softmax_forward against gemm_forward followed by softmax_forward over the
 last axis (reference: tensor_ops.c:1167-1228 then :1231-1270), bit for bit on both
-outputs: the k-split path whose reduction takes the softmax (the config-5 head,
-[64,512] x [1000,512]^T with a per-column bias), shapes that run the two calls
-(no split, rows longer than one block), scalar and absent biases, alpha / beta
-other than 1, and rows with infinite and NaN logits."""
+outputs: the k-split path whose reduction takes the softmax (the slices_* cases, one for
+each of the row kernels that read slices), shapes that run the two calls (few rows, the
+[64,512] x [1000,512]^T classifier head among them, and rows longer than one block), scalar
+and absent biases, alpha / beta other than 1, and rows with infinite and NaN logits."""
 import ctypes
 
 import numpy as np
@@ -22,6 +22,15 @@ CASES = [
     ("split_scalar_bias_nonfinite", 64, 512, 1000, "one", 1.0, 1.0, True),
     ("no_split_small", 8, 64, 100, "col", 1.0, 1.0, False),
     ("rows_past_block", 16, 512, 1500, "col", 1.0, 1.0, False),
+    # more than 64 rows, a k split and at most 1024 columns: 16 lanes, a wave, 256 and
+    # 1024 threads per row of slices
+    ("slices_16", 70, 1024, 16, "col", 1.0, 1.0, False),
+    ("slices_30_no_bias", 70, 1024, 30, None, 0.5, 1.0, True),
+    ("slices_200_scalar_bias", 65, 1024, 200, "one", 1.0, 1.0, True),
+    ("slices_400_alpha_beta", 1100, 1024, 400, "col", 0.75, -1.5, False),
+    ("slices_300_alpha_beta", 100, 512, 300, "one", 0.75, -1.5, True),
+    ("slices_1000", 70, 512, 1000, "col", 1.0, 1.0, True),
+    ("slices_1000_many_rows", 600, 512, 1000, None, 1.0, 1.0, True),
 ]
 
 

@@ -303,7 +303,8 @@ def test_capture_first_on_fresh_stream(hip, oracle_lib):
     """Calls captured on a stream the library has never used, with no eager call
     before them: Softmax over few long rows and DynamicQuantizeLinear (partials
     in the fixed capture workspaces), the no-allocation DynamicQuantizeLinear
-    and a Gemm whose eager plan splits k (captured unsplit).  Nothing may
+    and a Gemm whose eager plan splits k (captured unsplit; 70 rows, past the
+    few-rows kernel).  Nothing may
     allocate inside the capture; the graph is replayed on changed inputs and
     every replay is compared with eager calls on the same inputs (bit for bit;
     the Gemm against the oracle within tolerance, its eager plan differing)."""
@@ -320,16 +321,16 @@ def test_capture_first_on_fresh_stream(hip, oracle_lib):
         with torch.cuda.stream(side):
             sm_x = torch.empty((64, 32000), dtype=torch.float32, device="cuda")
             dq_x = torch.empty((8, 512, 1024), dtype=torch.float32, device="cuda")
-            ga = torch.empty((64, 512), dtype=torch.float32, device="cuda")
+            ga = torch.empty((70, 512), dtype=torch.float32, device="cuda")
             gb = torch.from_numpy(rng.normal(0, 0.05, (1000, 512)).astype(np.float32)).cuda()
             gc = torch.from_numpy(rng.normal(0, 1, (1, 1000)).astype(np.float32)).cuda()
-            outs = {"softmax": torch.empty_like(sm_x), "gemm": torch.empty((64, 1000), dtype=torch.float32, device="cuda")}
+            outs = {"softmax": torch.empty_like(sm_x), "gemm": torch.empty((70, 1000), dtype=torch.float32, device="cuda")}
             for k in ("dql", "dql_noalloc"):
                 outs[k] = torch.empty((8, 512, 1024), dtype=torch.uint8, device="cuda")
                 outs[k + "_scale"] = torch.empty([1], dtype=torch.float32, device="cuda")
                 outs[k + "_zp"] = torch.empty([1], dtype=torch.uint8, device="cuda")
             t = {"sm_x": wrap(sm_x, [64, 32000], O.F32), "dq_x": wrap(dq_x, [8, 512, 1024], O.F32),
-                 "ga": wrap(ga, [64, 512], O.F32), "gb": wrap(gb, [1000, 512], O.F32), "gc": wrap(gc, [1, 1000], O.F32)}
+                 "ga": wrap(ga, [70, 512], O.F32), "gb": wrap(gb, [1000, 512], O.F32), "gc": wrap(gc, [1, 1000], O.F32)}
             dts = {"softmax": O.F32, "gemm": O.F32, "dql": O.U8, "dql_noalloc": O.U8}
             for k, v in outs.items():
                 dt = dts.get(k, O.F32 if k.endswith("scale") else O.U8)
@@ -354,7 +355,7 @@ def test_capture_first_on_fresh_stream(hip, oracle_lib):
         for r in range(3):
             sm_np = rng.normal(0, 3 + r, (64, 32000)).astype(np.float32)
             dq_np = rng.normal(0, 0.5 + r, (8, 512, 1024)).astype(np.float32)
-            ga_np = rng.normal(0, 1, (64, 512)).astype(np.float32)
+            ga_np = rng.normal(0, 1, (70, 512)).astype(np.float32)
             sm_x.copy_(torch.from_numpy(sm_np))
             dq_x.copy_(torch.from_numpy(dq_np))
             ga.copy_(torch.from_numpy(ga_np))

@@ -118,3 +118,28 @@ def test_small_results_only(rec):
     """The runtime's copy is the slower one up to 16 KB only."""
     assert kernels(rec.to_host((4096,), O.F32, owned=True)) == ["k_result"]
     assert kernels(rec.to_host((16385,), O.U8, owned=True)) == []
+
+
+def test_gpu_cases_reach_their_kernels(rec):
+    """The GPU tests' cases named for a k split, a ring of LDS slots or a tile shape take it."""
+    from tests import test_gpu_conv_f16, test_gpu_gemm_f16_layouts, test_gpu_gemm_softmax
+    slices = [c for c in test_gpu_gemm_softmax.CASES if c[0].startswith("slices")]
+    rows = {16: "k_softmax_wave<1, 16,", 30: "k_softmax_wave<2, 16,", 200: "k_softmax_wave<4, 64,", 300: "k_softmax_row<1, 1024,",
+            400: "k_softmax_wave<8, 64,", 1000: "k_softmax_row<1, 1024,"}
+    for name, m, k, n, *_ in slices:
+        (gemm, softmax), err = rec.gemm_softmax(m, n, k)
+        want = "k_softmax_row<4, 256," if m == 600 else rows[n]
+        assert not err and gemm.kernel.startswith("k_gemm_f32_nt") and softmax.kernel.startswith(want), name
+        assert softmax.kernel.endswith("SmSlices>"), name
+    assert kernels(rec.gemm(70, 1000, 512)) == ["k_gemm_f32_nt", "k_splitk_reduce"]       # the capture tests' Gemm
+    for case in test_gpu_conv_f16.CASES:
+        name, xs, m, k, pads, strides, dil, group = case
+        if name.startswith(("ring", "tiles")):
+            launches, err = rec.conv(xs, m, k, pads, strides, dil, group, dt=O.F16)
+            bm, bp = name.split("_")[1].split("x")
+            assert not err and launches[-1].kernel.startswith(f"k_convh<{bm}, {bp},"), name
+    for m, n, k in test_gpu_gemm_f16_layouts.TILES:
+        for ta in (0, 1):
+            launches, err = rec.gemm(m, n, k, ta, 0, O.F16)
+            want = "k_convh<128, 128," if m > 2000 else "k_convh<64, 128,"
+            assert not err and launches[-1].kernel.startswith(want), (m, n, k)

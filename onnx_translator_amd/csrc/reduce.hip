@@ -499,12 +499,15 @@ bool launch_split(const void* x, int dtx, void* y, int dty, int64_t L, int G, di
 // times with dependent strided loads and left maps of few columns on a few CUs:
 // [8, 256, 1024] f32 241 -> 8.1 us, [4, 500, 16] 418 -> 8.6 us.  Axes of up to 64
 // values take 64 columns x 4 rows: 32 x 32 blocks would leave most rows of threads
-// one value or none ([64, 21, 4096]: 97 us, 12.3 us so).
+// one value or none ([64, 21, 4096]: 97 us, 12.3 us so).  Axes of one or two values take
+// 256 columns x 1 row and no LDS: 64 x 4 would leave two or three rows of threads without a
+// value ([64, 1, 16384] 10.7 against 7.1 us, [64, 2, 16384] 11.8 against 10.6, one thread per
+// column each time).
 template <int IPT, int CX, int CY, int DIN, int DOUT>
 __global__ __launch_bounds__(CX * CY) void k_softmax_cols(const void* __restrict__ X, int dtx, void* __restrict__ Y,
                                                                int dty, int64_t L, int64_t inner, int64_t r0,
                                                                uint32_t nbx) {
-    __shared__ double red[CY][CX];
+    __shared__ double red[CY > 1 ? CY : 1][CY > 1 ? CX : 1];
     const int cx = threadIdx.x & (CX - 1), ry = threadIdx.x / CX;
     const int64_t bo = blockIdx.x / nbx;
     const int64_t r = r0 + (int64_t)(blockIdx.x - bo * nbx) * CX + cx;
@@ -526,15 +529,17 @@ __global__ __launch_bounds__(CX * CY) void k_softmax_cols(const void* __restrict
             mx = w > mx ? w : mx;
         }
     }
-    red[ry][cx] = mx;
-    __syncthreads();
-    mx = -DBL_MAX;
+    if constexpr (CY > 1) {
+        red[ry][cx] = mx;
+        __syncthreads();
+        mx = -DBL_MAX;
 #pragma unroll
-    for (int i = 0; i < CY; i++) {
-        const double w = red[i][cx];
-        mx = w > mx ? w : mx;
+        for (int i = 0; i < CY; i++) {
+            const double w = red[i][cx];
+            mx = w > mx ? w : mx;
+        }
+        __syncthreads();
     }
-    __syncthreads();
     double sum = 0.0;
     if constexpr (IPT > 0) {
 #pragma unroll
@@ -545,11 +550,13 @@ __global__ __launch_bounds__(CX * CY) void k_softmax_cols(const void* __restrict
     } else {
         for (int64_t j = ry; j < L; j += CY) sum += sm_exp(ldx<DIN>(X, base + j * inner, dtx) - mx);
     }
-    red[ry][cx] = sum;
-    __syncthreads();
-    sum = 0.0;
+    if constexpr (CY > 1) {
+        red[ry][cx] = sum;
+        __syncthreads();
+        sum = 0.0;
 #pragma unroll
-    for (int i = 0; i < CY; i++) sum += red[i][cx];
+        for (int i = 0; i < CY; i++) sum += red[i][cx];
+    }
     if (!live) return;
     const double rs = 1.0 / sum;
     if constexpr (IPT > 0) {
@@ -566,8 +573,8 @@ __global__ __launch_bounds__(CX * CY) void k_softmax_cols(const void* __restrict
 
 template <int DIN, int DOUT>
 void launch_cols(const void* x, int dtx, void* y, int dty, int64_t outer, int64_t L, int64_t inner, hipStream_t s) {
-    const bool few = L <= 64;
-    const int cx = few ? 64 : 32, cy = few ? 4 : 32;
+    const bool one = L <= 2, few = L <= 64;
+    const int cx = one ? 256 : few ? 64 : 32, cy = one ? 1 : few ? 4 : 32;
     const int64_t ipt = (L + cy - 1) / cy;
     const dim3 b(cx * cy);
     // One grid dimension holds every (outer, column block).  The runtime takes fewer than 2^32
@@ -583,7 +590,8 @@ void launch_cols(const void* x, int dtx, void* y, int dty, int64_t outer, int64_
         char* yo = (char*)y + (size_t)(o * L * inner) * dt_bytes(dty);
 #define SM_COLS(I, CX, CY) \
     hipLaunchKernelGGL((k_softmax_cols<I, CX, CY, DIN, DOUT>), g, b, 0, s, xo, dtx, yo, dty, L, inner, r0, nbx)
-        if (few) {
+        if (one) SM_COLS(2, 256, 1);
+        else if (few) {
             if (ipt <= 2) SM_COLS(2, 64, 4);
             else if (ipt <= 4) SM_COLS(4, 64, 4);
             else if (ipt <= 8) SM_COLS(8, 64, 4);

@@ -16,7 +16,7 @@ pytestmark = pytest.mark.gpu
 ROWS = [(5, 1), (17, 16), (33, 17), (16, 32), (7, 33), (6, 64), (9, 65), (3, 256), (2, 257), (1025, 257), (1027, 321),
         (1024, 512), (1024, 513), (512, 1000), (511, 1000), (513, 1025), (512, 2048), (1024, 2049), (1023, 2049)]
 # outer, length, inner
-COLS = [(3, 1, 5), (2, 8, 63), (2, 9, 65), (1, 33, 64), (4, 64, 7), (2, 65, 33), (1, 128, 31), (1, 257, 32), (2, 512, 3),
+COLS = [(3, 1, 5), (2, 1, 257), (5, 2, 256), (3, 2, 300), (4, 3, 65), (2, 8, 63), (2, 9, 65), (1, 33, 64), (4, 64, 7), (2, 65, 33), (1, 128, 31), (1, 257, 32), (2, 512, 3),
         (1, 513, 40)]
 
 
@@ -81,7 +81,8 @@ def test_gemm_softmax_same_rows(hip, M, N):
 
 
 @pytest.mark.parametrize("shape,dtype", [((1 << 24, 2, 2), "float32"), (((1 << 22) + 3, 65, 1, 2), "float16"),
-                                         ((1, 2, (1 << 30) + 5), "float16")], ids=["outer24", "outer22", "inner30"])
+                                         ((1, 2, (1 << 30) + 5), "float16"),
+                                         ((1, 3, (1 << 29) + 5), "float16")], ids=["outer24", "outer22", "inner30", "inner29"])
 def test_softmax_columns_in_slices(hip, shape, dtype):
     """More column blocks than one launch holds, by the outer or the inner dimension: every
     value against torch's float32 softmax (1e-6 for f32 outputs of at most 1; one unit in the

@@ -32,16 +32,23 @@ def test_conv_f16_of_no_pixels(rec, h, w):
     assert r.returncode == 0, (r.returncode, r.stderr[-2000:])
 
 
-@pytest.mark.parametrize("shape,threads", [((1 << 24, 2, 2), 256), (((1 << 22) + 3, 65, 2), 1024), ((3, 2, (1 << 30) + 5), 256),
+@pytest.mark.parametrize("shape,threads", [((1 << 24, 2, 2), 256), (((1 << 22) + 3, 65, 2), 1024), ((3, 2, (1 << 30) + 5), 256), ((3, 3, (1 << 30) + 5), 256),
                                            ((2, 70, 1 << 28), 1024)], ids=lambda v: str(v))
 def test_softmax_columns_in_slices(rec, shape, threads):
     """Along an inner dimension: every column block launched once, within the runtime's
     2^32 work-items per dimension (the recorder refuses more, as the runtime does)."""
     launches, err = rec.softmax(shape, 1, O.F16)
     assert not err, err
-    cols = 64 if threads == 256 else 32
+    cols = 32 if threads == 1024 else 256 if shape[1] <= 2 else 64
     assert all(l.block == threads for l in launches)
     assert sum(l.grid[0] for l in launches) == shape[0] * -(-shape[2] // cols)
+
+
+def test_softmax_columns_of_two_values(rec):
+    """Every thread has a column: 256 of them per block."""
+    for length, cols in ((1, 256), (2, 256), (3, 64)):
+        (l,), err = rec.softmax((64, length, 16384), 1)
+        assert not err and l.grid[0] == 64 * 16384 // cols and l.block == 256
 
 
 # f32: direct 1x1, 64x64, 128x256, 64x256 and per-pixel plans, all with slices of k

@@ -104,15 +104,22 @@ template <int DOUT> __device__ __forceinline__ void sm_store(void* Y, int64_t i,
     else stx<DOUT>(Y, i, v, dty);
 }
 
-// A row's values in double: of a plain tensor, or (SmSlices, below) the k slices
-// of a Gemm.
+// A thread's values j0, j0 + STEP, ... of a row (`none` past its end and in a row that is
+// not live): of a plain tensor, or (SmSlices, below) of the k slices of a Gemm.
 template <int DIN> struct SmRows {
     // values that a float holds exactly are compared as floats
     using T = std::conditional_t<DIN == kF32 || DIN == kF16, float, double>;
     const void* X;
     int dtx;
     int64_t L;
-    __device__ __forceinline__ T operator()(int64_t row, int j) const { return (T)ldx<DIN>(X, row * L + j, dtx); }
+    template <int V, int STEP>
+    __device__ __forceinline__ void load(T (&x)[V], int64_t row, int j0, bool live, T none) const {
+#pragma unroll
+        for (int t = 0; t < V; t++) {
+            const int j = j0 + t * STEP;
+            x[t] = live && j < L ? (T)ldx<DIN>(X, row * L + j, dtx) : none;
+        }
+    }
 };
 
 // One block of T threads per row (inner == 1), the row kept in registers (IPT per
@@ -126,12 +133,9 @@ __global__ __launch_bounds__(T) void k_softmax_row(SRC src, void* __restrict__ Y
     __shared__ double lds[kW];
     const int64_t row = blockIdx.x;
     V x[IPT], m = kNone;
+    src.template load<IPT, T>(x, row, threadIdx.x, true, kNone);
 #pragma unroll
-    for (int t = 0; t < IPT; t++) {
-        const int j = threadIdx.x + t * T;
-        x[t] = j < L ? src(row, j) : kNone;
-        m = x[t] > m ? x[t] : m;
-    }
+    for (int t = 0; t < IPT; t++) m = x[t] > m ? x[t] : m;
     m = block_reduce<true, kW>(m, ldm);
     // the reference's maximum starts at -DBL_MAX: what a row of -inf (or NaN) keeps
     const double mx = m > kNone ? (double)m : -DBL_MAX;
@@ -620,11 +624,7 @@ __global__ __launch_bounds__(256) void k_softmax_wave(SRC src, void* __restrict_
     const int64_t row = (int64_t)blockIdx.x * kRows + threadIdx.x / GL;
     const bool live = row < outer;              // (every lane takes part in the reductions)
     T x[VPT], m = kNone;
-#pragma unroll
-    for (int t = 0; t < VPT; t++) {
-        const int j = l + t * GL;
-        x[t] = (live && j < L) ? src(row, j) : kNone;
-    }
+    src.template load<VPT, GL>(x, row, l, live, kNone);
 #pragma unroll
     for (int t = 0; t < VPT; t++) m = x[t] > m ? x[t] : m;
     m = lanes_allreduce<GL>(m, [](T a, T b) { return b > a ? b : a; });
@@ -681,7 +681,8 @@ bool launch_block_rows(const SRC& src, void* y, int dty, int64_t outer, int L, h
     // 11.0 us, [700, 700] 5.5 -> 3.7 us; at [600, 4096] the two forms took 9.2 and
     // 9.5 us, so the longer rows only with four of them per CU.
     if (L <= 4096 && outer >= (L <= 2048 ? 2 : 4) * num_cus()) {
-        if (L <= 1024) SM_ROW(4, 256);
+        if (L <= 512) SM_ROW(2, 256);
+        else if (L <= 1024) SM_ROW(4, 256);
         else if (L <= 2048) SM_ROW(8, 256);
         else SM_ROW(16, 256);
         return true;
@@ -1084,7 +1085,9 @@ __global__ __launch_bounds__(kGapSmallThreads) void k_gap_small_f32(const float*
 // takes them (double sum in slice order, alpha * acc + beta * c, rounded to f32),
 // written to Y as the logit; the rows then run as softmax_forward runs them: both
 // outputs equal the two launches they replace bit for bit.  cmode: 0 no bias, 1
-// one value, 2 per column, 3 per row.
+// one value, 2 per column, 3 per row.  All of a thread's values of four slices are read
+// before any logit is stored: value by value, each waited for its slices again, which made
+// [70, 1024] x [1024, 100] 15.6 us, 10.0 so ([1100, 1024] x [1024, 400] 34.5 -> 23.8).
 struct SmSlices {
     const float* part;
     int nsplit;
@@ -1095,15 +1098,31 @@ struct SmSlices {
     int cmode;
     float* Y;
     using T = float;
-    __device__ __forceinline__ float operator()(int64_t m, int j) const {
-        const int64_t i = m * N + j;
-        double acc = 0.0;
-        for (int sp = 0; sp < nsplit; sp++) acc += (double)part[(int64_t)sp * mn + i];
-        double r = alpha * acc;
-        if (cmode) r += beta * (double)c[cmode == 1 ? 0 : (cmode == 2 ? j : (int)m)];
-        const float y = (float)r;
-        Y[i] = y;
-        return y;
+    template <int V, int STEP>
+    __device__ __forceinline__ void load(float (&x)[V], int64_t m, int j0, bool live, float none) const {
+        const float* p = part + (live ? m : 0) * N;
+        int at[V];
+        double acc[V];
+#pragma unroll
+        for (int t = 0; t < V; t++) {
+            at[t] = min(j0 + t * STEP, N - 1);
+            acc[t] = 0.0;
+        }
+#pragma unroll 4
+        for (int sp = 0; sp < nsplit; sp++) {
+#pragma unroll
+            for (int t = 0; t < V; t++) acc[t] += (double)p[at[t]];
+            p += mn;
+        }
+#pragma unroll
+        for (int t = 0; t < V; t++) {
+            const int j = j0 + t * STEP;
+            x[t] = none;
+            if (!live || j >= N) continue;
+            double r = alpha * acc[t];
+            if (cmode) r += beta * (double)c[cmode == 1 ? 0 : (cmode == 2 ? j : (int)m)];
+            Y[m * N + j] = x[t] = (float)r;
+        }
     }
 };
 

@@ -40,7 +40,7 @@ struct ConvH {
     int HW, NHW;
     uint32_t rb;                             // bytes of a pixel's chunks: group * C8 * 16
     uint32_t xbytes, wbytes;
-    FastDiv fd_hw, fd_ohw, fd_ow, fd_c8, fd_kw, fd_khw, fd_g8;
+    FastDiv fd_hw, fd_ohw, fd_ow, fd_c8, fd_kw, fd_khw;
 };
 
 // ---- layout: X -> [N * H * W][group][C8] chunks, W -> [M][KHW][C8] chunks --------------
@@ -407,6 +407,23 @@ void launch_tiles_h(const TilesH& t, const uint4* xp, const uint4* wp, const Epi
     else launch_tiles<64, 64, kRing64x64, GEMM>(xp, wp, epi, y, dty, part, g, t.split, total, s);
 }
 
+// Layers that the general kernel (k_conv_mfma_f32, which gathers halves one by one) does
+// faster: so few products per output and so few channels out that the chunk copies of X
+// and 64-channel tiles are most of the work here, over enough pixels to fill the chip; with
+// few pixels its one pass over k per block is the slower one.  A stride past the window
+// copies pixels that no output uses, so more layers are among them.
+// Measured, general kernel -> this: [8, C, 256, 256] 1x1, C = 8 to one channel 35 -> 61 us, to
+// eight 46 -> 61, to 16 61 -> 63; C = 16 to eight 54 -> 65, 3x3 C = 2 to eight 68 -> 62; at
+// [16, 8, 64, 64] to eight channels 14.2 -> 11.5.  Stride 2: C = 16 to 16 24 -> 31, C = 32 to
+// eight 29 -> 33, C = 32 to 32 43 -> 34.  Planes too wide for the depthwise kernel, [1, 2,
+// 2000, 2000] 3x3: 495 -> 753.
+bool few_products(const ConvGeom& g) {
+    const int64_t K = (int64_t)g.Cg * g.KH * g.KW, P = (int64_t)g.N * g.OH * g.OW, NHW = (int64_t)g.N * g.H * g.W;
+    if (std::max(P, NHW / 4) * g.group <= 65536) return false;
+    const bool skips = g.sh > g.KH || g.sw > g.KW;
+    return (K <= 16 && g.Mg <= (skips || g.Cg == 1 ? 16 : 8)) || (skips && K <= 32 && g.Mg <= 8);
+}
+
 }  // namespace
 
 bool launch_conv_f16(const void* x, const void* w, const void* b, int dtb, void* y, int dty, const ConvGeom& cg,
@@ -416,6 +433,7 @@ bool launch_conv_f16(const void* x, const void* w, const void* b, int dtb, void*
     if (cg.N < 1 || cg.Cg < 1 || cg.H < 1 || cg.W < 1 || cg.KH < 1 || cg.KW < 1 || cg.group > 65535) return false;
     // the layout copies live in a workspace, which a captured call may not take
     if (stream_capturing(s)) return false;
+    if (few_products(cg)) return false;
     ConvH g;
     const int64_t C8 = (cg.Cg + 7) / 8, KHW = (int64_t)cg.KH * cg.KW, KC = KHW * C8;
     const int64_t NHW = (int64_t)cg.N * cg.H * cg.W, P = (int64_t)cg.N * cg.OH * cg.OW;

@@ -101,15 +101,15 @@ def test_gemm_f16_in_place_under_capture(rec, m, n, k):
         rec.capturing(False)
 
 
-@pytest.mark.parametrize("k,pads,dil", [((31, 31), 15, 1), ((2, 2), 25, 50)], ids=["31x31", "dilated"])
+@pytest.mark.parametrize("k", [31, 17])
 @pytest.mark.parametrize("dt", [O.F32, O.F16, O.U8], ids=["f32", "f16", "codes"])
-def test_depthwise_launch_within_the_work_items(rec, k, pads, dil, dt):
+def test_depthwise_launch_within_the_work_items(rec, k, dt):
     """Many planes of one pixel under a wide window, few to a block: the depthwise kernel's
     blocks would be past 2^32 work-items; the layer runs all the same."""
-    pads = (pads,) * 4
-    r = rec.conv((1 << 28, 1, 1, 1), 1, k, pads, (1, 1), (dil, dil), 1, dt=dt, codes=O.U8 if dt == O.U8 else None)
+    args, codes = (1, (k, k), (k // 2,) * 4), O.U8 if dt == O.U8 else None
+    r = rec.conv((1 << 28, 1, 1, 1), *args, dt=dt, codes=codes)
     assert len(kernels(r)) == 1
-    few = rec.conv((1 << 10, 1, 1, 1), 1, k, pads, (1, 1), (dil, dil), 1, dt=dt, codes=O.U8 if dt == O.U8 else None)
+    few = rec.conv((1 << 10, 1, 1, 1), *args, dt=dt, codes=codes)
     assert kernels(few) == ["k_conv_dw"]
 
 
@@ -125,6 +125,20 @@ def test_small_results_only(rec):
     """The runtime's copy is the slower one up to 16 KB only."""
     assert kernels(rec.to_host((4096,), O.F32, owned=True)) == ["k_result"]
     assert kernels(rec.to_host((16385,), O.U8, owned=True)) == []
+
+
+# x shape, output channels, window, stride, groups; whether the channels-last copies are taken
+F16_FEW = [((8, 8, 256, 256), 8, 1, 1, 1, 0), ((8, 16, 256, 256), 8, 1, 1, 1, 0), ((8, 16, 256, 256), 16, 1, 1, 1, 1),
+           ((8, 2, 256, 256), 8, 3, 1, 1, 1), ((16, 8, 64, 64), 8, 1, 1, 1, 1), ((16, 256, 28, 28), 256, 1, 1, 32, 0),
+           ((8, 16, 256, 256), 16, 1, 2, 1, 0), ((8, 32, 256, 256), 8, 1, 2, 1, 0), ((8, 32, 256, 256), 32, 1, 2, 1, 1),
+           ((1, 2, 2000, 2000), 2, 3, 1, 2, 0), ((32, 64, 56, 56), 64, 3, 1, 1, 1)]
+
+
+@pytest.mark.parametrize("xs,m,k,s,group,copies", F16_FEW, ids=lambda v: str(v).replace(" ", ""))
+def test_conv_f16_few_products(rec, xs, m, k, s, group, copies):
+    """f16 layers of few products per output over many pixels: the kernel without copies."""
+    names = kernels(rec.conv(xs, m, (k, k), (k // 2,) * 4, (s, s), group=group, dt=O.F16))
+    assert names[-1] == ("k_convh" if copies else "k_conv_mfma_f32")
 
 
 def test_gpu_cases_reach_their_kernels(rec):

@@ -47,9 +47,8 @@ template <int XQ> __device__ __forceinline__ float xq_value(uint32_t code, float
 // layer is outside the plan.
 bool launch_conv_depthwise(const void* x, int dtx, const void* w, const void* b, int dtb, void* y, int dty,
                            const ConvGeom& g, const ConvEpi& epi, const ConvXQ& xq, hipStream_t s);
-// The layers launch_conv_depthwise takes, by their shape alone.
-bool conv_depthwise_shape(const ConvGeom& g);
-
+// The layers launch_conv_depthwise takes, by their shape and whether X is f16 alone.
+bool conv_depthwise_shape(const ConvGeom& g, bool half);
 // float16 X and W on the f16 matrix cores (convh.hip): f16 / f32 output, f32 / f16 or
 // no bias, any groups.  False, with nothing launched and no error, when the layer is outside
 // the plan or there is no memory for the copies.

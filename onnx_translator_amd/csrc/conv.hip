@@ -1442,7 +1442,7 @@ bool conv_entry(const char* name, const Tensor* X, const Tensor* W, const Tensor
             const ConvEpi epi{(const float*)z, relu, fq};
             const ConvXQ xq{(const float*)xsd, xzd};
             bool fq_applied = false;
-            const bool dw = conv_depthwise_shape(g) &&
+            const bool dw = conv_depthwise_shape(g, false) &&
                             launch_conv_depthwise(x, xq_kind == 1 ? kU8 : kI8, w, b, dtb, y, dty, g, epi, xq, s);
             if (dw) fq_applied = fq_kind != 0;
             const bool ok = dw ? true : xq_kind == 1 ? launch_conv_tiled_xq<1>(x, w, b, dtb, y, dty, g, epi, xq, s, &fq_applied)
@@ -1454,7 +1454,7 @@ bool conv_entry(const char* name, const Tensor* X, const Tensor* W, const Tensor
         } else if (!exact_mode() && !big && g.Kg > 0 && f32_exact_dtype(dtx) && f32_exact_dtype(dtw)) {
             const bool same = dtx == dtw && (dtx == kF32 || dtx == kF16);
             const ConvEpi no_epi{nullptr, 0, FakeQuant{nullptr, nullptr, nullptr, nullptr, 0}};
-            if (same && conv_depthwise_shape(g)) {
+            if (same && conv_depthwise_shape(g, dtx == kF16)) {
                 const bool epi_ok = dty == kF32 && (!has_b || dtb == kF32);
                 const ConvEpi epi{(const float*)z, relu, fq};
                 if (launch_conv_depthwise(x, dtx, w, b, dtb, y, dty, g, epi_ok ? epi : no_epi,

@@ -166,7 +166,22 @@ constexpr int kDwR3 = 7, kDwR5 = 4;
 // channel, 3x3: 16 outputs 7.6 -> 4.6 us, 32 6.9 against 7.6, 64 10.9 against 11.4).
 constexpr int kDwMaxMult = 16;
 
-bool dw_plan(const ConvGeom& g, PlaneTiles& p) {
+// Strides past the window stage rows and columns that no output uses (a plane's tiles
+// whole, once per output channel), where the implicit GEMM gathers what it needs.  A pixel
+// of one group costs that about as much as 28 + 1.6 KH KW staged values (twice as many with
+// f16 operands, which it decodes); a plane's second and further reads, from L2, count 0.6.
+// Measured on both sides of the line, GEMM -> this, [32, 64, 112, 112] f32: 1x1 stride 5
+// 27 -> 23 us, stride 6 20 -> 24, stride 8 12.4 -> 20.5; 3x3 stride 6 29 -> 23, stride 8
+// 19 -> 23; four output channels per input channel, 16 -> 64: 1x1 stride 3 24 -> 21, stride
+// 4 15 -> 25, stride 8 6.4 -> 20.8; sixteen, 4 -> 64: 3x3 stride 2 25 -> 22.  f16: 1x1 stride
+// 8 23 -> 18; four, 1x1 stride 4 33 -> 23, stride 6 14.6 -> 21.8; sixteen, 3x3 stride 3
+// 24 -> 30.
+bool dw_pays(const ConvGeom& g, const PlaneTiles& p, bool half) {
+    const double staged = (double)p.PR * p.PW * p.tiles / ((double)g.OH * g.OW);
+    return (0.4 + 0.6 * g.Mg) * staged <= (28.0 + 1.6 * g.KH * g.KW) * (half ? 2.1 : 1.0);
+}
+
+bool dw_plan(const ConvGeom& g, bool half, PlaneTiles& p) {
     if (g.Cg != 1 || g.Mg > kDwMaxMult || g.KH < 1 || g.KW < 1 || g.sh < 1 || g.sw < 1 || g.dh < 1 || g.dw < 1) return false;
     const int64_t reach = (int64_t)1 << 29;              // elements: byte offsets stay below 2^31
     const int64_t planes = (int64_t)g.N * g.M;
@@ -178,7 +193,7 @@ bool dw_plan(const ConvGeom& g, PlaneTiles& p) {
     p.C = g.C; p.H = g.H; p.W = g.W; p.OH = g.OH; p.OW = g.OW; p.M = g.M; p.KH = g.KH; p.KW = g.KW;
     p.pt = g.pt; p.pl = g.pl; p.sh = g.sh; p.sw = g.sw; p.dh = g.dh; p.dw = g.dw;
     p.planes = (int)planes;
-    return plan_planes(p, R, g.KH * g.KW);
+    return plan_planes(p, R, g.KH * g.KW) && dw_pays(g, p, half);
 }
 
 template <int DT, int ODT>
@@ -194,9 +209,9 @@ void launch_dw_window(const void* x, const void* w, const void* b, int dtb, void
 
 }  // namespace
 
-bool conv_depthwise_shape(const ConvGeom& g) {
+bool conv_depthwise_shape(const ConvGeom& g, bool half) {
     PlaneTiles p;
-    return dw_plan(g, p);
+    return dw_plan(g, half, p);
 }
 
 bool launch_conv_depthwise(const void* x, int dtx, const void* w, const void* b, int dtb, void* y, int dty,
@@ -204,7 +219,7 @@ bool launch_conv_depthwise(const void* x, int dtx, const void* w, const void* b,
     const bool codes = dtx == kU8 || dtx == kI8;
     if ((dtx != kF32 && dtx != kF16 && !codes) || (codes && dty != kF32) || (dty != kF32 && dty != kF16) || (b && dtb != kF32 && dtb != kF16)) return false;
     PlaneTiles p;
-    if (!dw_plan(g, p)) return false;
+    if (!dw_plan(g, dtx == kF16, p)) return false;
     p.xbytes = (uint32_t)((int64_t)g.N * g.C * g.H * g.W * (codes ? 1 : dtx == kF16 ? 2 : 4));
     if (dtx == kU8) launch_dw_window<kU8, kF32>(x, w, b, dtb, y, p, epi, xq, s);
     else if (dtx == kI8) launch_dw_window<kI8, kF32>(x, w, b, dtb, y, p, epi, xq, s);

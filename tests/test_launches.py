@@ -141,6 +141,20 @@ def test_conv_f16_few_products(rec, xs, m, k, s, group, copies):
     assert names[-1] == ("k_convh" if copies else "k_conv_mfma_f32")
 
 
+# channels, output channels, window, stride; which kernel f32 and codes take, which f16 takes
+DW_STRIDES = [(64, 64, 1, 5, 1, 1), (64, 64, 1, 6, 0, 1), (64, 64, 1, 8, 0, 1), (64, 64, 3, 6, 1, 1), (64, 64, 3, 8, 0, 1),
+              (16, 64, 1, 3, 1, 1), (16, 64, 1, 4, 0, 1), (16, 64, 1, 6, 0, 0), (16, 64, 3, 4, 0, 1), (16, 64, 5, 8, 0, 0),
+              (4, 64, 3, 2, 1, 1), (4, 64, 3, 3, 0, 0), (64, 64, 16, 16, 1, 1), (16, 64, 3, 2, 1, 1), (16, 256, 3, 1, 1, 1)]
+
+
+@pytest.mark.parametrize("c,m,k,s,f32,f16", DW_STRIDES, ids=lambda v: str(v))
+def test_depthwise_strides(rec, c, m, k, s, f32, f16):
+    """Strides well past the window: the gathering kernels, for f32 and its codes alike."""
+    for dt, codes, dw in ((O.F32, None, f32), (O.F32, O.I8, f32), (O.F16, None, f16)):
+        names = kernels(rec.conv((32, c, 112, 112), m, (k, k), (k // 2,) * 4, (s, s), (1, 1), c, dt=dt, codes=codes))
+        assert ("k_conv_dw" in names) == bool(dw), names
+
+
 def test_gpu_cases_reach_their_kernels(rec):
     """The GPU tests' cases named for a k split, a ring of LDS slots or a tile shape take it."""
     from tests import test_gpu_conv_f16, test_gpu_gemm_f16_layouts, test_gpu_gemm_softmax

@@ -959,7 +959,21 @@ void launch_planes(const float* x, float* y, const PlaneTiles& p, hipStream_t s)
     else hipLaunchKernelGGL((k_maxpool_planes<K, S, R, false>), grid, blk, lds, s, x, y, p);
 }
 
-// The plans above; false: another window, or a tensor past their 32-bit offsets.
+// Planes too wide for one chunk of columns per thread are staged chunk after chunk, each
+// waited for: with few tiles to a CU nothing covers that, and a wave per output row
+// (k_maxpool_rows) is done sooner.  Measured, rows -> tiles: 3x3 stride 1 [1, 16, 33, 33]
+// 4.1 -> 5.8 us, [1, 64, 128, 128] (320 tiles) 6.9 -> 7.4, [4, 64, 64, 64] (512) 7.2 -> 6.0,
+// one chunk [1, 64, 50, 50] 4.2 -> 4.6, [4, 64, 50, 50] 6.3 -> 4.9; 5x5 (25 values per output
+// there) [1, 64, 33, 33] 6.0 -> 6.6, [1, 64, 64, 64] the same.  2x2 stride 2 uses no value
+// twice: [4, 64, 128, 128] padded by one 7.3 -> 9.5, [32, 64, 112, 112] 33 -> 28.
+bool pool_few_tiles(const PlaneTiles& p) {
+    const int64_t blocks = (p.planes + (int64_t)p.np - 1) / p.np * p.tiles, cus = num_cus();
+    if (p.KH == 2 && p.sh == 2 && p.PW > 64) return blocks <= 8 * cus;
+    if (p.KH > 3) return p.cc > 1 && 2 * blocks < cus;
+    return p.cc > 1 ? blocks < 2 * cus : p.PW > 32 && 2 * blocks < cus;
+}
+
+// The plans above; false: another window, few tiles, or a tensor past their 32-bit offsets.
 bool launch_maxpool_f32(const float* x, float* y, const PoolGeom& g, int64_t planes, hipStream_t s) {
     const int64_t reach = (int64_t)1 << 29;       // elements: byte offsets stay below 2^31
     if (planes * g.H * g.W >= reach || planes * g.OH * g.OW >= reach || planes >= reach) return false;
@@ -981,7 +995,7 @@ bool launch_maxpool_f32(const float* x, float* y, const PoolGeom& g, int64_t pla
     p.pt = g.pt; p.pl = g.pl; p.sh = g.sh; p.sw = g.sw; p.dh = g.dh; p.dw = g.dw;
     p.planes = (int)planes;
     p.xbytes = (uint32_t)(planes * g.H * g.W * 4);
-    if (!plan_planes(p, kPoolStripRows, 0)) return false;
+    if (!plan_planes(p, kPoolStripRows, 0) || pool_few_tiles(p)) return false;
     if (g.KH == 2) g.sh == 1 ? launch_planes<2, 1>(x, y, p, s) : launch_planes<2, 2>(x, y, p, s);
     else if (g.KH == 3) g.sh == 1 ? launch_planes<3, 1>(x, y, p, s) : launch_planes<3, 2>(x, y, p, s);
     else g.sh == 1 ? launch_planes<5, 1>(x, y, p, s) : launch_planes<5, 2>(x, y, p, s);

@@ -121,6 +121,14 @@ class Recorder:
                              self.tensor((1,), codes), wt, b, O.PT(), 0, y, ctypes.byref(p))
         return self.call("conv2d_forward", self.tensor(xs, dt), wt, b, y, ctypes.byref(p))
 
+    def maxpool(self, xs, k, stride, pad):
+        n, c, h, w = xs
+        out = [(v + 2 * pad - k) // stride + 1 for v in (h, w)]
+        keep = [O._ints((pad,) * 4), O._ints((stride,) * 2), O._ints((1, 1)), O._ints((k, k))]
+        p = O.CPoolParams()
+        p.pads, p.strides, p.dilations, p.kernel_shape = [ctypes.cast(v, ctypes.POINTER(ctypes.c_int)) for v in keep]
+        return self.call("max_pool_forward", self.tensor(xs, O.F32), self.tensor([n, c] + out, O.F32), ctypes.byref(p))
+
     def gemm(self, m, n, k, ta=0, tb=1, dt=O.F32, bias=True):
         a, b = self.tensor((k, m) if ta else (m, k), dt), self.tensor((n, k) if tb else (k, n), dt)
         return self.call("gemm_forward", a, b, self.tensor((n,), O.F32) if bias else O.PT(), self.tensor((m, n), dt),

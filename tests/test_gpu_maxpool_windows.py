@@ -17,6 +17,11 @@ CASES = [((1, 1, 1, 1), 3, 1, (1, 1, 1, 1)), ((3, 70, 7, 7), 3, 1, (1, 1, 1, 1))
          ((2, 3, 17, 18), 2, 2, (1, 1, 1, 1)), ((2, 3, 18, 18), 2, 2, (0, 0, 0, 0)), ((2, 7, 19, 17), 2, 2, (0, 0, 0, 0)),
          ((1, 5, 33, 1026), 2, 2, (0, 0, 0, 0)), ((1, 2, 9, 1000), 3, 1, (1, 1, 1, 1)), ((1, 3, 6, 6), 3, 2, (4, 4, 4, 4)),
          ((2, 3, 18, 19), 2, 2, (0, 0, 1, 1))]
+# wide planes, enough of them for the row tiles: several tiles per plane and chunks per row
+TILES = [((8, 20, 150, 131), 3, 1, (1, 1, 1, 1)), ((2, 65, 57, 55), 3, 2, (1, 1, 1, 1)), ((2, 65, 58, 56), 3, 2, (0, 0, 0, 0)),
+         ((1, 66, 100, 64), 5, 2, (2, 2, 2, 2)), ((1, 260, 9, 1000), 3, 1, (1, 1, 1, 1)), ((4, 600, 20, 130), 2, 2, (1, 1, 1, 1)),
+         ((3, 100, 70, 75), 2, 1, (0, 0, 0, 0))]
+CASES += TILES
 
 
 @pytest.mark.parametrize("shape,k,s,pads", CASES, ids=["x".join(map(str, c[0])) + f"_k{c[1]}s{c[2]}p{c[3][0]}{c[3][2]}" for c in CASES])

@@ -155,9 +155,22 @@ def test_depthwise_strides(rec, c, m, k, s, f32, f16):
         assert ("k_conv_dw" in names) == bool(dw), names
 
 
+# x shape, window, stride, pad; whether the row tiles are taken
+POOLS = [((1, 16, 33, 33), 3, 1, 1, 0), ((1, 64, 128, 128), 3, 1, 1, 0), ((4, 64, 64, 64), 3, 1, 1, 1), ((1, 64, 50, 50), 3, 1, 1, 0),
+         ((4, 64, 50, 50), 3, 1, 1, 1), ((4, 64, 28, 28), 3, 1, 1, 1), ((1, 64, 100, 100), 2, 1, 0, 0), ((4, 64, 100, 100), 2, 1, 0, 1),
+         ((1, 64, 33, 33), 5, 1, 2, 0), ((1, 64, 64, 64), 5, 1, 2, 1), ((1, 16, 7, 7), 5, 1, 2, 1), ((4, 64, 128, 128), 2, 2, 1, 0),
+         ((32, 64, 112, 112), 2, 2, 1, 1), ((4, 64, 33, 33), 3, 2, 0, 0), ((8, 128, 33, 33), 3, 2, 0, 1)]
+
+
+@pytest.mark.parametrize("xs,k,s,p,tiles", POOLS, ids=lambda v: str(v).replace(" ", ""))
+def test_maxpool_few_tiles(rec, xs, k, s, p, tiles):
+    """Few tiles of wide planes: a wave per output row."""
+    assert kernels(rec.maxpool(xs, k, s, p)) == ["k_maxpool_planes" if tiles else "k_maxpool_rows"]
+
+
 def test_gpu_cases_reach_their_kernels(rec):
     """The GPU tests' cases named for a k split, a ring of LDS slots or a tile shape take it."""
-    from tests import test_gpu_conv_f16, test_gpu_gemm_f16_layouts, test_gpu_gemm_softmax
+    from tests import test_gpu_conv_f16, test_gpu_gemm_f16_layouts, test_gpu_gemm_softmax, test_gpu_maxpool_windows
     slices = [c for c in test_gpu_gemm_softmax.CASES if c[0].startswith("slices")]
     rows = {16: "k_softmax_wave<1, 16,", 30: "k_softmax_wave<2, 16,", 200: "k_softmax_wave<4, 64,", 300: "k_softmax_row<1, 1024,",
             400: "k_softmax_wave<8, 64,", 1000: "k_softmax_row<1, 1024,"}
@@ -178,3 +191,5 @@ def test_gpu_cases_reach_their_kernels(rec):
             launches, err = rec.gemm(m, n, k, ta, 0, O.F16)
             want = "k_convh<128, 128," if m > 2000 else "k_convh<64, 128,"
             assert not err and launches[-1].kernel.startswith(want), (m, n, k)
+    for xs, k, stride, pads in test_gpu_maxpool_windows.TILES:
+        assert kernels(rec.maxpool(xs, k, stride, pads[0])) == ["k_maxpool_planes"], xs

@@ -2,7 +2,7 @@
 //
 // tensor_ops/tensor_ops.c:1167-1228 accumulates sum_k A'[m,k] B'[k,n] in
 // double, sequentially in k, then adds beta * C with the reference's bias
-// broadcast rules and writes through the output encoder.  Three kernels:
+// broadcast rules and writes through the output encoder.  The kernels:
 //
 //  * k_gemm_mfma_f32 — v_mfma_f32_32x32x2f32 (fp32 operands, fp32 accumulate),
 //    for the layouts (transA = 1) and dtypes k_gemm_f32_nt does not take.
@@ -18,7 +18,7 @@
 //    (dequantised while staging) or f32 B [K, N]: v_mfma_f32_32x32x2f32,
 //    128x256x16 tiles over 8 waves, split-K with a deterministic reduction for
 //    small grids.
-//  * k_gemm_rows — the same operands with at most 64 rows of A and B [N, K]: one
+//  * k_gemm_rows — the same operands with few rows of A (few_rows) and B [N, K]: one
 //    pass over B straight into the MFMA operands.
 //  * convh.hip's f16 GEMM — small f16 grids, and the other f16 layouts and sizes through
 //    copies of the operands in rows of 16-byte chunks.
@@ -1018,11 +1018,11 @@ __global__ __launch_bounds__(256) void k_splitk_reduce(GemmArgs g, const float* 
 // k = 16 h + e in every group, A and B alike), so B is read once, without LDS, 64 (codes)
 // or 256 (f32) contiguous bytes of a row per wave and chunk (a second chunk in flight per
 // wave measured the same or slower: the other waves' loads are in flight anyway).  The
-// waves' sums meet in LDS and are added in wave order in double.  One launch, no workspace.  The order of the sums depends on K and the number
-// of waves (from N and K) only, and the codes' values are DequantizeLinear's bits (as in
-// k_gemm_f32_nt), so the fused and the unfused weight-only-quantized Gemm agree bit for
-// bit.  128-row tiles with a k split took these before: A [8, 4096] x int8 [4096, 4096]
-// 45 -> MEASW us.
+// waves' sums meet in LDS and are added in wave order in double.  One launch, no workspace.
+// The order of the sums depends on K and the number of waves only (from N, K and whether M
+// is past 32), and the codes' values are DequantizeLinear's bits (as in k_gemm_f32_nt), so
+// the fused and the unfused weight-only-quantized Gemm agree bit for bit.  128-row tiles with
+// a k split took these before: A [8, 4096] x int8 [4096, 4096] 45 -> 9.4 us.
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 
 template <int MT, int YDT, int BQ>
@@ -1250,13 +1250,23 @@ void launch_nt_kernel(const GemmArgs& g, const WoqB& q, int kchunk, int nsplit, 
     launch_nt_kernel_kt<BM, BN, BK, WGM, WGN, BQ, SPLIT, KN, false>(g, q, kchunk, nsplit, ydt, s);
 }
 
-// Few rows: k_gemm_rows up to 32.  Up to 64 (four row tiles, 64 MFMAs per chunk and wave)
-// where the waves have few chunks each or the columns fill the chip; else the 128-row tiles
-// with their k split are as good: [64, 512] x [1000, 512] 10.5 -> 8.0 us, [48, 4096] x int8
-// [4096, 4096] 46.7 -> 29.5, but [64, 4096] x [4096, 4096] 42.3 against 43.1, [62, 4016] x
-// [344, 4016] 22.3 against 31.1.
+// Few rows: k_gemm_rows, whose blocks of 16 columns each run through all of k, against the
+// 128-row tiles, whose k splits up to 16 ways.  Up to 16 rows always (f32 [16, 25088] x [256,
+// 25088] 83 us on tiles, 91 so, but with int8 codes 75 and 58; both must run one schedule, or the
+// fused and the unfused weight-only-quantized Gemm would differ).  With 17 to 32 rows the split wins for
+// long k while all its slices run at once, on one block per CU (N <= 1024) or two, by M K:
+// tiles -> rows, f32 [32, K] x [1000, K] K = 2048 14.8 -> 13.2, 4096 20.3 -> 23.7, 9216 37 ->
+// 51; [24, 4096] 20.4 -> 21.4; [32, 6144] x [2048, 6144] 35 -> 35; [32, 25088] x [4096, 25088]
+// 244 -> 153; int8 [32, 9216] x [1000, 9216] 34 -> 39.  Up to 64 rows (four row tiles, 64 MFMAs per
+// chunk and wave) for K <= 1024, of few columns by M K again ([64, 512] x [1000, 512] 10.5
+// -> 8.0 us, gemm_softmax_forward [64, 1024] x [100, 1024] 12.7 -> 14.8), and 48 rows of any
+// depth where the columns fill the chip ([48, 4096] x int8 [4096, 4096] 46.7 -> 29.5).
 inline bool few_rows(int M, int N, int K) {
-    return M <= 32 || (M <= 64 && K <= 1024) || (M <= 48 && (N + 15) / 16 >= num_cus());
+    const int64_t mk = (int64_t)M * K, slices = (int64_t)((N + 63) / 64) * 16, cus = num_cus();
+    if (M <= 16) return true;
+    if (M <= 32) return slices > 2 * cus || mk <= (slices > cus ? 192 << 10 : 96 << 10);
+    if (M <= 64 && K <= 1024) return slices > cus || mk <= 48 << 10;
+    return M <= 48 && (N + 15) / 16 >= cus;
 }
 
 template <int MT, int BQ>

@@ -14,7 +14,8 @@ from tests.helpers import assert_close
 pytestmark = pytest.mark.gpu
 
 SHAPES = [(1, 1, 4), (1, 1000, 512), (15, 17, 60), (16, 16, 64), (17, 33, 68), (32, 40, 1028), (33, 48, 1024), (48, 4100, 132),
-          (64, 100, 1000), (3, 70, 4100), (48, 4096, 1100)]
+          (64, 100, 1000), (3, 70, 4100), (48, 4096, 1100),
+          (64, 100, 764)]
 BIAS = {"none": lambda m, n: None, "one": lambda m, n: (1,), "col": lambda m, n: (n,), "row": lambda m, n: (m, 1),
         "2d": lambda m, n: (m, n)}
 

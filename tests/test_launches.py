@@ -168,6 +168,19 @@ def test_maxpool_few_tiles(rec, xs, k, s, p, tiles):
     assert kernels(rec.maxpool(xs, k, s, p)) == ["k_maxpool_planes" if tiles else "k_maxpool_rows"]
 
 
+FEW_ROWS = [(1, 10, 100352, 1), (16, 256, 25088, 1), (32, 1000, 3072, 1), (32, 1000, 4096, 0), (24, 1000, 4096, 1), (24, 1000, 6144, 0),
+            (32, 64, 25088, 0), (32, 2048, 6144, 1), (32, 2048, 9216, 0), (32, 4096, 25088, 1), (64, 1000, 512, 1), (64, 1000, 1024, 0),
+            (64, 4096, 1024, 1), (48, 4096, 4096, 1), (48, 1000, 2048, 0), (64, 4096, 4096, 0), (64, 100, 764, 1), (65, 1000, 512, 0)]
+
+
+@pytest.mark.parametrize("m,n,k,rows", FEW_ROWS, ids=lambda v: str(v))
+def test_gemm_few_rows(rec, m, n, k, rows):
+    """Few rows against few columns and a long k: the tiles with their k split.  The same for
+    the weight's codes, which return the same bits."""
+    for names in (kernels(rec.gemm(m, n, k)), kernels(rec.woq(m, n, k))):
+        assert names[0] == ("k_gemm_rows" if rows else "k_gemm_f32_nt")
+
+
 def test_gpu_cases_reach_their_kernels(rec):
     """The GPU tests' cases named for a k split, a ring of LDS slots or a tile shape take it."""
     from tests import test_gpu_conv_f16, test_gpu_gemm_f16_layouts, test_gpu_gemm_softmax, test_gpu_maxpool_windows

@@ -121,12 +121,6 @@ def test_small_result_of_another_device(rec):
     assert kernels(rec.to_host((1000,), O.F32, device=-1)) == []
 
 
-def test_small_results_only(rec):
-    """The runtime's copy is the slower one up to 16 KB only."""
-    assert kernels(rec.to_host((4096,), O.F32, owned=True)) == ["k_result"]
-    assert kernels(rec.to_host((16385,), O.U8, owned=True)) == []
-
-
 # x shape, output channels, window, stride, groups; whether the channels-last copies are taken
 F16_FEW = [((8, 8, 256, 256), 8, 1, 1, 1, 0), ((8, 16, 256, 256), 8, 1, 1, 1, 0), ((8, 16, 256, 256), 16, 1, 1, 1, 1),
            ((8, 2, 256, 256), 8, 3, 1, 1, 1), ((16, 8, 64, 64), 8, 1, 1, 1, 1), ((16, 256, 28, 28), 256, 1, 1, 32, 0),

@@ -725,8 +725,11 @@ static bool sync_copy_under_capture(const char* name) {
 
 // Small results: a kernel writes them to pinned host memory (its own launch, in stream
 // order), the stream is waited for and the bytes are copied on.  The runtime's copy to
-// pageable memory goes through its staging and a copy engine instead: 4 KB 24 -> 14.6 us,
-// and 88 us less per forward of the one-image residual network with its two outputs.
+// pageable memory goes through its staging and a copy engine instead.  On an idle stream that
+// takes 22 us up to 16 KB and 10-20 us from there to 256 KB, against 13-14 and 14-23 so; behind
+// queued work, as results are read, the kernel is the faster one throughout: 88 us less per
+// forward of the one-image residual network (two results of 4 KB), 379 against 414 us for 64
+// images (two of 256,000 bytes).
 // Memory that is not the library's own may lie on another device, which a kernel here
 // cannot be sure to reach: the runtime's copy takes it.  False: not taken (nothing enqueued).
 constexpr size_t kSmallResult = 256 << 10;

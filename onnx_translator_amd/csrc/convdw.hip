@@ -168,17 +168,19 @@ constexpr int kDwMaxMult = 16;
 
 // Strides past the window stage rows and columns that no output uses (a plane's tiles
 // whole, once per output channel), where the implicit GEMM gathers what it needs.  A pixel
-// of one group costs that about as much as 28 + 1.6 KH KW staged values (twice as many with
-// f16 operands, which it decodes); a plane's second and further reads, from L2, count 0.6.
+// of one group costs that about as much as 28 + 1.75 KH KW staged values (2.5 times as many
+// with f16 operands, which it decodes); here a plane's second and further reads, from L2, count
+// 0.6, and a tap of the general form (R == 1) about 1 / 4.
 // Measured on both sides of the line, GEMM -> this, [32, 64, 112, 112] f32: 1x1 stride 5
 // 27 -> 23 us, stride 6 20 -> 24, stride 8 12.4 -> 20.5; 3x3 stride 6 29 -> 23, stride 8
 // 19 -> 23; four output channels per input channel, 16 -> 64: 1x1 stride 3 24 -> 21, stride
-// 4 15 -> 25, stride 8 6.4 -> 20.8; sixteen, 4 -> 64: 3x3 stride 2 25 -> 22.  f16: 1x1 stride
-// 8 23 -> 18; four, 1x1 stride 4 33 -> 23, stride 6 14.6 -> 21.8; sixteen, 3x3 stride 3
-// 24 -> 30.
-bool dw_pays(const ConvGeom& g, const PlaneTiles& p, bool half) {
-    const double staged = (double)p.PR * p.PW * p.tiles / ((double)g.OH * g.OW);
-    return (0.4 + 0.6 * g.Mg) * staged <= (28.0 + 1.6 * g.KH * g.KW) * (half ? 2.1 : 1.0);
+// 4 15 -> 25, stride 8 6.4 -> 20.8, 7x7 stride 2 146 -> 105; eight, 8 -> 64, 7x7 stride 4
+// 28 -> 39; sixteen, 4 -> 64: 3x3 stride 2 25 -> 22; int8 codes 5x5 stride 8 29 -> 22.  f16: 1x1 stride 8 23 -> 18; four, 1x1
+// stride 4 33 -> 23, stride 6 14.6 -> 21.8; eight, 3x3 stride 4 28 -> 21; sixteen, 3x3 stride
+// 3 24 -> 30.
+bool dw_pays(const ConvGeom& g, const PlaneTiles& p, int R, bool half) {
+    const double staged = (double)p.PR * p.PW * p.tiles / ((double)g.OH * g.OW), taps = (double)g.KH * g.KW;
+    return (0.4 + 0.6 * g.Mg) * staged + (R == 1 ? 0.26 * g.Mg * taps : 0.0) <= (28.0 + 1.75 * taps) * (half ? 2.5 : 1.0);
 }
 
 bool dw_plan(const ConvGeom& g, bool half, PlaneTiles& p) {
@@ -193,7 +195,7 @@ bool dw_plan(const ConvGeom& g, bool half, PlaneTiles& p) {
     p.C = g.C; p.H = g.H; p.W = g.W; p.OH = g.OH; p.OW = g.OW; p.M = g.M; p.KH = g.KH; p.KW = g.KW;
     p.pt = g.pt; p.pl = g.pl; p.sh = g.sh; p.sw = g.sw; p.dh = g.dh; p.dw = g.dw;
     p.planes = (int)planes;
-    return plan_planes(p, R, g.KH * g.KW) && dw_pays(g, p, half);
+    return plan_planes(p, R, g.KH * g.KW) && dw_pays(g, p, R, half);
 }
 
 template <int DT, int ODT>

@@ -410,18 +410,25 @@ void launch_tiles_h(const TilesH& t, const uint4* xp, const uint4* wp, const Epi
 // Layers that the general kernel (k_conv_mfma_f32, which gathers halves one by one) does
 // faster: so few products per output and so few channels out that the chunk copies of X
 // and 64-channel tiles are most of the work here, over enough pixels to fill the chip; with
-// few pixels its one pass over k per block is the slower one.  A stride past the window
-// copies pixels that no output uses, so more layers are among them.
+// few pixels its one pass over k per block is the slower one.  1x1 windows with a stride
+// copy pixels that no output uses, so more layers are among them, as are the depthwise
+// ones whose stride is past the window (seven of a chunk's eight channels are padding).
 // Measured, general kernel -> this: [8, C, 256, 256] 1x1, C = 8 to one channel 35 -> 61 us, to
 // eight 46 -> 61, to 16 61 -> 63; C = 16 to eight 54 -> 65, 3x3 C = 2 to eight 68 -> 62; at
-// [16, 8, 64, 64] to eight channels 14.2 -> 11.5.  Stride 2: C = 16 to 16 24 -> 31, C = 32 to
-// eight 29 -> 33, C = 32 to 32 43 -> 34.  Planes too wide for the depthwise kernel, [1, 2,
-// 2000, 2000] 3x3: 495 -> 753.
+// [16, 8, 64, 64] to eight channels 14.2 -> 11.5; eight groups [8, 8, 128, 128] to eight
+// channels each 87 -> 102, 16 channels to eight 125 -> 102.  Stride 2: C = 16 to 16 24 -> 31,
+// C = 32 to eight 29 -> 33, C = 32 to 32 43 -> 34; stride 4 C = 16 to 16 21 -> 20.  Planes too
+// wide for the depthwise kernel, [1, 2, 2000, 2000] 3x3: 495 -> 753; [32, 16, 112, 112] to 64 by
+// groups of one, 5x5 stride 8: 26 -> 71.
 bool few_products(const ConvGeom& g) {
-    const int64_t K = (int64_t)g.Cg * g.KH * g.KW, P = (int64_t)g.N * g.OH * g.OW, NHW = (int64_t)g.N * g.H * g.W;
-    if (std::max(P, NHW / 4) * g.group <= 65536) return false;
-    const bool skips = g.sh > g.KH || g.sw > g.KW;
-    return (K <= 16 && g.Mg <= (skips || g.Cg == 1 ? 16 : 8)) || (skips && K <= 32 && g.Mg <= 8);
+    const int64_t K = (int64_t)g.Cg * g.KH * g.KW, pixels = (int64_t)g.N * g.OH * g.OW * g.group;
+    const bool point = g.KH == 1 && g.KW == 1 && (g.sh > 1 || g.sw > 1);
+    // (a stride's copies count as a quarter of the work that their pixels would be)
+    const int64_t work = point ? std::max(pixels, (int64_t)g.N * g.H * g.W / 4 * g.group) : pixels;
+    const bool skips = point || (g.Cg == 1 && (g.sh > g.KH || g.sw > g.KW));
+    const int64_t most = skips && g.Mg <= 8 ? 32 : g.group == 1 || g.Cg == 1 ? 16 : 8;
+    if (g.Mg <= 8) return K <= most && work > 65536;
+    return g.Mg <= 16 && K <= most && (point || g.Cg == 1) && pixels > 65536;
 }
 
 }  // namespace

@@ -1256,15 +1256,15 @@ void launch_nt_kernel(const GemmArgs& g, const WoqB& q, int kchunk, int nsplit, 
 // fused and the unfused weight-only-quantized Gemm would differ).  With 17 to 32 rows the split wins for
 // long k while all its slices run at once, on one block per CU (N <= 1024) or two, by M K:
 // tiles -> rows, f32 [32, K] x [1000, K] K = 2048 14.8 -> 13.2, 4096 20.3 -> 23.7, 9216 37 ->
-// 51; [24, 4096] 20.4 -> 21.4; [32, 6144] x [2048, 6144] 35 -> 35; [32, 25088] x [4096, 25088]
-// 244 -> 153; int8 [32, 9216] x [1000, 9216] 34 -> 39.  Up to 64 rows (four row tiles, 64 MFMAs per
+// 51; [24, 4096] 20.4 -> 21.4; [32, K] x [2048, K] K = 9216 47 -> 51, 16384 75 -> 87; [32, 25088]
+// x [4096, 25088] 244 -> 153; int8 [32, 9216] x [1000, 9216] 34 -> 39, x [2048, 9216] 48 -> 38.  Up to 64 rows (four row tiles, 64 MFMAs per
 // chunk and wave) for K <= 1024, of few columns by M K again ([64, 512] x [1000, 512] 10.5
 // -> 8.0 us, gemm_softmax_forward [64, 1024] x [100, 1024] 12.7 -> 14.8), and 48 rows of any
 // depth where the columns fill the chip ([48, 4096] x int8 [4096, 4096] 46.7 -> 29.5).
 inline bool few_rows(int M, int N, int K) {
     const int64_t mk = (int64_t)M * K, slices = (int64_t)((N + 63) / 64) * 16, cus = num_cus();
     if (M <= 16) return true;
-    if (M <= 32) return slices > 2 * cus || mk <= (slices > cus ? 192 << 10 : 96 << 10);
+    if (M <= 32) return slices > 2 * cus || mk <= (slices > cus ? 320 << 10 : 96 << 10);
     if (M <= 64 && K <= 1024) return slices > cus || mk <= 48 << 10;
     return M <= 48 && (N + 15) / 16 >= cus;
 }

@@ -104,8 +104,8 @@ template <int DOUT> __device__ __forceinline__ void sm_store(void* Y, int64_t i,
     else stx<DOUT>(Y, i, v, dty);
 }
 
-// A thread's values j0, j0 + STEP, ... of a row (`none` past its end and in a row that is
-// not live): of a plain tensor, or (SmSlices, below) of the k slices of a Gemm.
+// A thread's values j0, j0 + STEP, ... of a row of n (`none` past its end and in a row that
+// is not live): of a plain tensor, or (SmSlices, below) of the k slices of a Gemm.
 template <int DIN> struct SmRows {
     // values that a float holds exactly are compared as floats
     using T = std::conditional_t<DIN == kF32 || DIN == kF16, float, double>;
@@ -113,11 +113,11 @@ template <int DIN> struct SmRows {
     int dtx;
     int64_t L;
     template <int V, int STEP>
-    __device__ __forceinline__ void load(T (&x)[V], int64_t row, int j0, bool live, T none) const {
+    __device__ __forceinline__ void load(T (&x)[V], int64_t row, int j0, bool live, int n, T none) const {
 #pragma unroll
         for (int t = 0; t < V; t++) {
             const int j = j0 + t * STEP;
-            x[t] = live && j < L ? (T)ldx<DIN>(X, row * L + j, dtx) : none;
+            x[t] = live && j < n ? (T)ldx<DIN>(X, row * L + j, dtx) : none;
         }
     }
 };
@@ -133,7 +133,7 @@ __global__ __launch_bounds__(T) void k_softmax_row(SRC src, void* __restrict__ Y
     __shared__ double lds[kW];
     const int64_t row = blockIdx.x;
     V x[IPT], m = kNone;
-    src.template load<IPT, T>(x, row, threadIdx.x, true, kNone);
+    src.template load<IPT, T>(x, row, threadIdx.x, true, L, kNone);
 #pragma unroll
     for (int t = 0; t < IPT; t++) m = x[t] > m ? x[t] : m;
     m = block_reduce<true, kW>(m, ldm);
@@ -624,7 +624,7 @@ __global__ __launch_bounds__(256) void k_softmax_wave(SRC src, void* __restrict_
     const int64_t row = (int64_t)blockIdx.x * kRows + threadIdx.x / GL;
     const bool live = row < outer;              // (every lane takes part in the reductions)
     T x[VPT], m = kNone;
-    src.template load<VPT, GL>(x, row, l, live, kNone);
+    src.template load<VPT, GL>(x, row, l, live, L, kNone);
 #pragma unroll
     for (int t = 0; t < VPT; t++) m = x[t] > m ? x[t] : m;
     m = lanes_allreduce<GL>(m, [](T a, T b) { return b > a ? b : a; });
@@ -961,16 +961,18 @@ void launch_planes(const float* x, float* y, const PlaneTiles& p, hipStream_t s)
 
 // Planes too wide for one chunk of columns per thread are staged chunk after chunk, each
 // waited for: with few tiles to a CU nothing covers that, and a wave per output row
-// (k_maxpool_rows) is done sooner.  Measured, rows -> tiles: 3x3 stride 1 [1, 16, 33, 33]
-// 4.1 -> 5.8 us, [1, 64, 128, 128] (320 tiles) 6.9 -> 7.4, [4, 64, 64, 64] (512) 7.2 -> 6.0,
-// one chunk [1, 64, 50, 50] 4.2 -> 4.6, [4, 64, 50, 50] 6.3 -> 4.9; 5x5 (25 values per output
-// there) [1, 64, 33, 33] 6.0 -> 6.6, [1, 64, 64, 64] the same.  2x2 stride 2 uses no value
-// twice: [4, 64, 128, 128] padded by one 7.3 -> 9.5, [32, 64, 112, 112] 33 -> 28.
+// (k_maxpool_rows) is done sooner, up to about 64 rows of 64 outputs per CU (10 with 25 values
+// per output).  Measured, rows -> tiles: 3x3 stride 1 [1, 16, 33, 33] 4.1 -> 5.8 us, [1, 64, 128,
+// 128] (320 tiles) 6.9 -> 7.4, [4, 64, 64, 64] (512) 7.2 -> 6.0, [1, 3, 1000, 1000] 44 -> 24, one
+// chunk [1, 64, 50, 50] 4.2 -> 4.6, [4, 64, 50, 50] 6.3 -> 4.9; 5x5 [1, 64, 33, 33] 6.0 -> 6.6,
+// [1, 64, 64, 64] the same, [1, 16, 128, 128] 9.1 -> 7.2.  2x2 stride 2 uses no value twice:
+// [4, 64, 128, 128] padded by one 7.3 -> 9.5, [32, 64, 112, 112] 33 -> 28.
 bool pool_few_tiles(const PlaneTiles& p) {
-    const int64_t blocks = (p.planes + (int64_t)p.np - 1) / p.np * p.tiles, cus = num_cus();
-    if (p.KH == 2 && p.sh == 2 && p.PW > 64) return blocks <= 8 * cus;
-    if (p.KH > 3) return p.cc > 1 && 2 * blocks < cus;
-    return p.cc > 1 ? blocks < 2 * cus : p.PW > 32 && 2 * blocks < cus;
+    const int64_t tiles = (p.planes + (int64_t)p.np - 1) / p.np * p.tiles, cus = num_cus();
+    const int64_t rows = (int64_t)p.planes * p.OH * ((p.OW + 63) / 64);
+    if (p.KH == 2 && p.sh == 2 && p.PW > 64) return tiles <= 8 * cus;
+    if (p.KH > 3) return p.cc > 1 && 2 * tiles < cus && rows <= 10 * cus;
+    return (p.cc > 1 ? tiles < 2 * cus : p.PW > 32 && 2 * tiles < cus) && rows <= 64 * cus;
 }
 
 // The plans above; false: another window, few tiles, or a tensor past their 32-bit offsets.
@@ -1113,13 +1115,13 @@ struct SmSlices {
     float* Y;
     using T = float;
     template <int V, int STEP>
-    __device__ __forceinline__ void load(float (&x)[V], int64_t m, int j0, bool live, float none) const {
+    __device__ __forceinline__ void load(float (&x)[V], int64_t m, int j0, bool live, int n, float none) const {
         const float* p = part + (live ? m : 0) * N;
         int at[V];
         double acc[V];
 #pragma unroll
         for (int t = 0; t < V; t++) {
-            at[t] = min(j0 + t * STEP, N - 1);
+            at[t] = min(j0 + t * STEP, n - 1);
             acc[t] = 0.0;
         }
 #pragma unroll 4
@@ -1132,7 +1134,7 @@ struct SmSlices {
         for (int t = 0; t < V; t++) {
             const int j = j0 + t * STEP;
             x[t] = none;
-            if (!live || j >= N) continue;
+            if (!live || j >= n) continue;
             double r = alpha * acc[t];
             if (cmode) r += beta * (double)c[cmode == 1 ? 0 : (cmode == 2 ? j : (int)m)];
             Y[m * N + j] = x[t] = (float)r;

@@ -124,7 +124,8 @@ def test_small_result_of_another_device(rec):
 # x shape, output channels, window, stride, groups; whether the channels-last copies are taken
 F16_FEW = [((8, 8, 256, 256), 8, 1, 1, 1, 0), ((8, 16, 256, 256), 8, 1, 1, 1, 0), ((8, 16, 256, 256), 16, 1, 1, 1, 1),
            ((8, 2, 256, 256), 8, 3, 1, 1, 1), ((16, 8, 64, 64), 8, 1, 1, 1, 1), ((16, 256, 28, 28), 256, 1, 1, 32, 0),
-           ((8, 16, 256, 256), 16, 1, 2, 1, 0), ((8, 32, 256, 256), 8, 1, 2, 1, 0), ((8, 32, 256, 256), 32, 1, 2, 1, 1),
+           ((8, 16, 256, 256), 16, 1, 2, 1, 0), ((8, 32, 256, 256), 8, 1, 2, 1, 0), ((8, 32, 256, 256), 32, 1, 2, 1, 1), ((8, 16, 256, 256), 16, 1, 4, 1, 1), ((8, 3, 256, 256), 8, 3, 8, 1, 1), ((32, 16, 112, 112), 64, 5, 8, 16, 0),
+           ((8, 128, 128, 128), 64, 1, 1, 8, 1), ((8, 64, 128, 128), 64, 1, 1, 8, 0),
            ((1, 2, 2000, 2000), 2, 3, 1, 2, 0), ((32, 64, 56, 56), 64, 3, 1, 1, 1)]
 
 
@@ -138,7 +139,7 @@ def test_conv_f16_few_products(rec, xs, m, k, s, group, copies):
 # channels, output channels, window, stride; which kernel f32 and codes take, which f16 takes
 DW_STRIDES = [(64, 64, 1, 5, 1, 1), (64, 64, 1, 6, 0, 1), (64, 64, 1, 8, 0, 1), (64, 64, 3, 6, 1, 1), (64, 64, 3, 8, 0, 1),
               (16, 64, 1, 3, 1, 1), (16, 64, 1, 4, 0, 1), (16, 64, 1, 6, 0, 0), (16, 64, 3, 4, 0, 1), (16, 64, 5, 8, 0, 0),
-              (4, 64, 3, 2, 1, 1), (4, 64, 3, 3, 0, 0), (64, 64, 16, 16, 1, 1), (16, 64, 3, 2, 1, 1), (16, 256, 3, 1, 1, 1)]
+              (8, 64, 7, 4, 0, 1), (8, 64, 3, 4, 0, 1), (64, 64, 5, 8, 1, 1), (4, 64, 3, 2, 1, 1), (4, 64, 3, 3, 0, 0), (64, 64, 16, 16, 1, 1), (16, 64, 3, 2, 1, 1), (16, 256, 3, 1, 1, 1)]
 
 
 @pytest.mark.parametrize("c,m,k,s,f32,f16", DW_STRIDES, ids=lambda v: str(v))
@@ -152,7 +153,7 @@ def test_depthwise_strides(rec, c, m, k, s, f32, f16):
 # x shape, window, stride, pad; whether the row tiles are taken
 POOLS = [((1, 16, 33, 33), 3, 1, 1, 0), ((1, 64, 128, 128), 3, 1, 1, 0), ((4, 64, 64, 64), 3, 1, 1, 1), ((1, 64, 50, 50), 3, 1, 1, 0),
          ((4, 64, 50, 50), 3, 1, 1, 1), ((4, 64, 28, 28), 3, 1, 1, 1), ((1, 64, 100, 100), 2, 1, 0, 0), ((4, 64, 100, 100), 2, 1, 0, 1),
-         ((1, 64, 33, 33), 5, 1, 2, 0), ((1, 64, 64, 64), 5, 1, 2, 1), ((1, 16, 7, 7), 5, 1, 2, 1), ((4, 64, 128, 128), 2, 2, 1, 0),
+         ((1, 64, 33, 33), 5, 1, 2, 0), ((1, 64, 64, 64), 5, 1, 2, 1), ((1, 16, 7, 7), 5, 1, 2, 1), ((1, 3, 1000, 1000), 3, 1, 1, 1), ((1, 16, 128, 128), 5, 1, 2, 1), ((4, 64, 128, 128), 2, 2, 1, 0),
          ((32, 64, 112, 112), 2, 2, 1, 1), ((4, 64, 33, 33), 3, 2, 0, 0), ((8, 128, 33, 33), 3, 2, 0, 1)]
 
 
@@ -163,7 +164,7 @@ def test_maxpool_few_tiles(rec, xs, k, s, p, tiles):
 
 
 FEW_ROWS = [(1, 10, 100352, 1), (16, 256, 25088, 1), (32, 1000, 3072, 1), (32, 1000, 4096, 0), (24, 1000, 4096, 1), (24, 1000, 6144, 0),
-            (32, 64, 25088, 0), (32, 2048, 6144, 1), (32, 2048, 9216, 0), (32, 4096, 25088, 1), (64, 1000, 512, 1), (64, 1000, 1024, 0),
+            (32, 64, 25088, 0), (32, 2048, 9216, 1), (32, 2048, 16384, 0), (32, 4096, 25088, 1), (64, 1000, 512, 1), (64, 1000, 1024, 0),
             (64, 4096, 1024, 1), (48, 4096, 4096, 1), (48, 1000, 2048, 0), (64, 4096, 4096, 0), (64, 100, 764, 1), (65, 1000, 512, 0)]
 
 

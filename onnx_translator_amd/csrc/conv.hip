@@ -10,10 +10,12 @@
 //    (c, kh, kw), MODE 1 1x1 float4, MODE 2 tap-blocked channels with
 //    b128 LDS reads), split-K for small grids, fused Relu / residual
 //    epilogue (described at the kernel and at launch_conv_tiled_xq).
-//  * convdw.hip — one input channel per group (depthwise), f32 or f16.
-//  * convh.hip — f16 input and weights on the f16 matrix cores.
-//  * k_conv_mfma_f32 — other fp32-exact dtypes (decoded while staging):
-//    implicit GEMM on v_mfma_f32_32x32x2f32.  Per group:
+//  * convdw.hip — one input channel per group (depthwise), f32, f16 or codes, but for
+//    strides well past the window.
+//  * convh.hip — f16 input and weights on the f16 matrix cores, but for few products
+//    per output over many pixels and under graph capture.
+//  * k_conv_mfma_f32 — those f16 layers and the other fp32-exact dtypes (decoded while
+//    staging): implicit GEMM on v_mfma_f32_32x32x2f32.  Per group:
 //    M = out channels, N = batch * OH * OW pixels, K = Cin/g * KH * KW.  The
 //    block tile is 64 channels x 256 pixels (4 waves side by side, each
 //    64 x 64 = 2x2 MFMA tiles), BK = 16.  Each thread owns one pixel column

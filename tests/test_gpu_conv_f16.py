@@ -26,6 +26,9 @@ CASES = [
     ("tiles_64x128", (8, 16, 56, 56), 72, (3, 3), (1, 1, 1, 1), (1, 1), (1, 1), 1),
     ("tiles_128x128", (24, 8, 54, 52), 130, (1, 1), (0, 0, 0, 0), (1, 1), (1, 1), 1),
     ("oh_odd_width2", (2, 16, 10, 5), 8, (3, 3), (1, 1, 1, 1), (1, 1), (1, 1), 1),
+    # few products per output over many pixels: the general kernel
+    ("few_products", (8, 9, 98, 95), 7, (1, 1), (0, 0, 0, 0), (1, 1), (1, 1), 1),
+    ("few_products_stride2", (8, 16, 190, 191), 16, (1, 1), (0, 0, 0, 0), (2, 2), (1, 1), 1),
     # many k-tiles through the rings of LDS slots: every remainder of three slots (18, 19 and
     # 20 tiles of 64x128) and of two (2 and 11 tiles of 128x128)
     ("ring_64x128_18", (32, 128, 28, 28), 128, (3, 3), (1, 1, 1, 1), (1, 1), (1, 1), 1),

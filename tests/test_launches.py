@@ -194,6 +194,8 @@ def test_gpu_cases_reach_their_kernels(rec):
             launches, err = rec.conv(xs, m, k, pads, strides, dil, group, dt=O.F16)
             bm, bp = name.split("_")[1].split("x")
             assert not err and launches[-1].kernel.startswith(f"k_convh<{bm}, {bp},"), name
+        elif name.startswith("few"):
+            assert kernels(rec.conv(xs, m, k, pads, strides, dil, group, dt=O.F16)) == ["k_conv_mfma_f32"], name
     for m, n, k in test_gpu_gemm_f16_layouts.TILES:
         for ta in (0, 1):
             launches, err = rec.gemm(m, n, k, ta, 0, O.F16)

@@ -2,6 +2,7 @@
 launches are recorded instead of run.  Tensors are headers over addresses that nothing reads."""
 import collections
 import ctypes
+import fcntl
 import os
 import subprocess
 
@@ -18,9 +19,16 @@ def _newer(path, sources):
 
 
 def build():
-    """Links (compiling what is stale) and returns the recording library's path."""
+    """Links (compiling what is stale) and returns the recording library's path; one process
+    at a time."""
     os.makedirs(os.path.dirname(OUT), exist_ok=True)
     os.makedirs(B.OBJ, exist_ok=True)
+    with open(OUT + ".lock", "w") as lock:
+        fcntl.flock(lock, fcntl.LOCK_EX)
+        return _build()
+
+
+def _build():
     headers = [os.path.join(B.CSRC, f) for f in os.listdir(B.CSRC) if f.endswith(".h")]
     stub = os.path.join(HERE, "hip_stub.cpp")
     objs = [os.path.join(B.OBJ, os.path.splitext(s)[0] + ".o") for s in B.SOURCES]
